@@ -130,6 +130,18 @@ struct SparHipNormSummary {
   int has_nan;
 };
 
+/* One tensor of spar_hip_launch_adamw_batch: its arrays of `count` contiguous
+ * elements and its own bias corrections. */
+struct SparHipAdamwTensor {
+  void* parameter;
+  const void* gradient;
+  void* first_moment;
+  void* second_moment;
+  uint64_t count;
+  double first_correction;
+  double second_correction;
+};
+
 /* ---------------------------------------------------------------- runtime */
 
 /* Number of visible HIP devices (replaces the cudaGetDeviceCount check in
@@ -546,10 +558,29 @@ struct SparHipStatus spar_hip_launch_gradient_norm_summary(struct SparHipNormSum
                                                            const void* gradient, uint64_t count,
                                                            int dtype, int device);
 
+/* The summaries of `tensor_count` gradients of one dtype into
+ * summaries[0 .. tensor_count) (device memory), each as above: gradient k has
+ * counts[k] contiguous elements at gradients[k] (the arrays of pointers and
+ * counts are host memory, read before the call returns).  Many gradients
+ * share a launch, so a model's small ones do not cost one each. */
+struct SparHipStatus spar_hip_launch_gradient_norm_summaries(struct SparHipNormSummary* summaries,
+                                                             const void* const* gradients,
+                                                             const uint64_t* counts,
+                                                             uint64_t tensor_count, int dtype,
+                                                             int device);
+
 /* values[i] = (T)((double)values[i] * factor) in place; factor must be
  * finite.  Replaces spar_cuda_launch_scale_in_place (cuda_kernels.hpp:121-122). */
 struct SparHipStatus spar_hip_launch_scale_in_place(void* values, uint64_t count, int dtype,
                                                     double factor, int device);
+
+/* The same for `tensor_count` arrays of one dtype, which must not overlap:
+ * counts[k] elements at values[k] (host arrays, read before the call
+ * returns). */
+struct SparHipStatus spar_hip_launch_scale_in_place_batch(void* const* values,
+                                                          const uint64_t* counts,
+                                                          uint64_t tensor_count, int dtype,
+                                                          double factor, int device);
 
 /* One AdamW step over `count` contiguous elements, in place on the parameter
  * and both moments, with the bias corrections 1 - beta^step supplied by the
@@ -564,6 +595,14 @@ struct SparHipStatus spar_hip_launch_adamw(void* parameter, const void* gradient
                                            double beta1, double beta2, double epsilon,
                                            double weight_decay, double first_correction,
                                            double second_correction, int device);
+
+/* The same step over `tensor_count` tensors of one dtype, which must not
+ * overlap (`tensors` is host memory, read before the call returns). */
+struct SparHipStatus spar_hip_launch_adamw_batch(const struct SparHipAdamwTensor* tensors,
+                                                 uint64_t tensor_count, int dtype,
+                                                 double learning_rate, double beta1,
+                                                 double beta2, double epsilon,
+                                                 double weight_decay, int device);
 
 /* ------------------------------------------------------ random generation */
 

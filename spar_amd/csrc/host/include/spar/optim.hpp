@@ -137,8 +137,8 @@ class AdamW {
   [[nodiscard]] const Entry* entry_of(const nn::Parameter& parameter) const noexcept;
   // Whether `entry` takes part in a step; throws if it cannot.
   [[nodiscard]] static bool steps(const Entry& entry);
-  // One fused update of `entry`'s Parameter and moments.
-  void update(Entry& entry) const;
+  // One update of the entries' Parameters and moments, batched by device and dtype.
+  void update(std::span<Entry* const> entries) const;
 
   std::vector<Entry> entries_;
   double learning_rate_;

@@ -2,10 +2,12 @@
 // tensors.  Names, validation order, messages and exception types are
 // Spar's (src/nn/parameter.cpp, src/optim/adamw.cpp,
 // src/training/gradients.cpp); the per-element work runs in the backend's
-// kernels (spar_hip_launch_adamw, spar_hip_launch_gradient_norm_summary,
-// spar_hip_launch_scale_in_place).  The norm enqueues every gradient's
-// summary before one read-back per device, where the reference synchronises
-// once per gradient (gradients.cpp:119).
+// kernels over whole parameter lists (spar_hip_launch_adamw_batch,
+// spar_hip_launch_gradient_norm_summaries,
+// spar_hip_launch_scale_in_place_batch), one call per device and dtype.  The
+// norm enqueues every gradient's summary before one read-back per device and
+// dtype, where the reference synchronises once per gradient
+// (gradients.cpp:119).
 #include "spar/optim.hpp"
 
 #include <algorithm>
@@ -191,18 +193,27 @@ class SummarySlots final {
   int device_;
 };
 
-// Summaries of the given gradients (all on `device`), computed into one
+// Tensors of one device and dtype, which one batched call takes.
+using GroupKey = std::pair<int, DType>;
+
+GroupKey group_of(const Tensor& tensor) { return {tensor.device().index(), tensor.dtype()}; }
+
+// Summaries of the given gradients (all of group `key`), computed into one
 // device array and read back with one copy.
 std::vector<SparHipNormSummary> device_summaries(const std::vector<const Tensor*>& gradients,
-                                                 int device) {
+                                                 const GroupKey& key) {
+  const int device{key.first};
   const SummarySlots slots{gradients.size(), device};
-  for (std::size_t k{0}; k < gradients.size(); ++k) {
-    const Tensor& gradient{*gradients[k]};
-    hip::check(spar_hip_launch_gradient_norm_summary(slots.at(k), HipTensorAccess::data(gradient),
-                                                     gradient.numel(),
-                                                     hip::dtype_tag(gradient.dtype()), device),
-               "global gradient norm", device);
+  std::vector<const void*> data;
+  std::vector<std::uint64_t> counts;
+  for (const Tensor* gradient : gradients) {
+    data.push_back(HipTensorAccess::data(*gradient));
+    counts.push_back(gradient->numel());
   }
+  hip::check(spar_hip_launch_gradient_norm_summaries(slots.at(0), data.data(), counts.data(),
+                                                     counts.size(), hip::dtype_tag(key.second),
+                                                     device),
+             "global gradient norm", device);
   std::vector<SparHipNormSummary> host(gradients.size());
   hip::check(spar_hip_copy_device_to_host(host.data(), slots.at(0),
                                           host.size() * sizeof(SparHipNormSummary), device),
@@ -214,15 +225,13 @@ std::vector<SparHipNormSummary> device_summaries(const std::vector<const Tensor*
 
 double global_grad_norm(std::span<nn::Parameter> parameters) {
   const std::vector<Tensor> gradients{checked_gradients(parameters, "global gradient norm")};
-  std::map<int, std::vector<std::size_t>> by_device;
-  for (std::size_t k{0}; k < gradients.size(); ++k) {
-    by_device[gradients[k].device().index()].push_back(k);
-  }
+  std::map<GroupKey, std::vector<std::size_t>> groups;
+  for (std::size_t k{0}; k < gradients.size(); ++k) groups[group_of(gradients[k])].push_back(k);
   std::vector<SparHipNormSummary> summaries(gradients.size());
-  for (const auto& [device, members] : by_device) {
+  for (const auto& [key, members] : groups) {
     std::vector<const Tensor*> group;
     for (const std::size_t k : members) group.push_back(&gradients[k]);
-    const auto results{device_summaries(group, device)};
+    const auto results{device_summaries(group, key)};
     for (std::size_t j{0}; j < members.size(); ++j) summaries[members[j]] = results[j];
   }
   NormTotal total;
@@ -233,11 +242,21 @@ double global_grad_norm(std::span<nn::Parameter> parameters) {
 void scale_gradients(std::span<nn::Parameter> parameters, double factor) {
   if (!std::isfinite(factor)) throw std::invalid_argument{"Gradient scale factor must be finite"};
   std::vector<Tensor> gradients{checked_gradients(parameters, "gradient scaling")};
+  struct Group {
+    std::vector<void*> values;
+    std::vector<std::uint64_t> counts;
+  };
+  std::map<GroupKey, Group> groups;
   for (Tensor& gradient : gradients) {
-    hip::check(spar_hip_launch_scale_in_place(HipTensorAccess::mutable_data(gradient),
-                                              gradient.numel(), hip::dtype_tag(gradient.dtype()),
-                                              factor, gradient.device().index()),
-               "gradient scaling", gradient.device());
+    Group& group{groups[group_of(gradient)]};
+    group.values.push_back(HipTensorAccess::mutable_data(gradient));
+    group.counts.push_back(gradient.numel());
+  }
+  for (const auto& [key, group] : groups) {
+    hip::check(spar_hip_launch_scale_in_place_batch(group.values.data(), group.counts.data(),
+                                                    group.counts.size(),
+                                                    hip::dtype_tag(key.second), factor, key.first),
+               "gradient scaling", key.first);
   }
 }
 
@@ -338,24 +357,36 @@ bool AdamW::steps(const Entry& entry) {
   return true;
 }
 
-void AdamW::update(Entry& entry) const {
-  State& state{*entry.state};
-  ++state.step;
-  Tensor value{entry.parameter.tensor().detach()};
-  const Tensor gradient{entry.parameter.grad()};
+// Steps the entries, the tensors of one device and dtype in one batched call.
+void AdamW::update(std::span<Entry* const> entries) const {
+  std::map<std::pair<int, DType>, std::vector<SparHipAdamwTensor>> groups;
   // Bias corrections computed on the host, as the reference's device path
-  // does (cuda_ops.cppm:675-676).
-  const auto correction = [step = static_cast<double>(state.step)](double beta) {
-    return 1.0 - std::pow(beta, step);
-  };
-  hip::check(spar_hip_launch_adamw(HipTensorAccess::mutable_data(value),
-                                   HipTensorAccess::data(gradient),
-                                   HipTensorAccess::mutable_data(state.first_moment),
-                                   HipTensorAccess::mutable_data(state.second_moment),
-                                   value.numel(), hip::dtype_tag(value.dtype()), learning_rate_,
-                                   beta1_, beta2_, epsilon_, weight_decay_, correction(beta1_),
-                                   correction(beta2_), value.device().index()),
-             "AdamW update", value.device());
+  // does (cuda_ops.cppm:675-676); most entries share a step count.
+  std::uint64_t step{0};
+  double first_correction{0.0};
+  double second_correction{0.0};
+  for (Entry* entry : entries) {
+    State& state{*entry->state};
+    ++state.step;
+    if (state.step != step) {
+      step = state.step;
+      first_correction = 1.0 - std::pow(beta1_, static_cast<double>(step));
+      second_correction = 1.0 - std::pow(beta2_, static_cast<double>(step));
+    }
+    Tensor value{entry->parameter.tensor().detach()};
+    const Tensor gradient{entry->parameter.grad()};
+    groups[{value.device().index(), value.dtype()}].push_back(SparHipAdamwTensor{
+        HipTensorAccess::mutable_data(value), HipTensorAccess::data(gradient),
+        HipTensorAccess::mutable_data(state.first_moment),
+        HipTensorAccess::mutable_data(state.second_moment), value.numel(), first_correction,
+        second_correction});
+  }
+  for (const auto& [key, tensors] : groups) {
+    hip::check(spar_hip_launch_adamw_batch(tensors.data(), tensors.size(),
+                                           hip::dtype_tag(key.second), learning_rate_, beta1_,
+                                           beta2_, epsilon_, weight_decay_, key.first),
+               "AdamW update", key.first);
+  }
 }
 
 // Every stepping entry is validated before anything changes, and the zero
@@ -374,7 +405,7 @@ void AdamW::step() {
                                            0});
   }
   for (auto& [entry, state] : first_states) entry->state.emplace(std::move(state));
-  for (Entry* entry : stepping) update(*entry);
+  update(stepping);
 }
 
 void AdamW::move_to(Device target) {

@@ -48,6 +48,13 @@ class NormSummary(ctypes.Structure):
                 ("has_infinity", ctypes.c_int), ("has_nan", ctypes.c_int)]
 
 
+class AdamwTensor(ctypes.Structure):
+    _fields_ = [("parameter", ctypes.c_void_p), ("gradient", ctypes.c_void_p),
+                ("first_moment", ctypes.c_void_p), ("second_moment", ctypes.c_void_p),
+                ("count", ctypes.c_uint64), ("first_correction", ctypes.c_double),
+                ("second_correction", ctypes.c_double)]
+
+
 class HipError(RuntimeError):
     def __init__(self, name: str, status: Status, message: str):
         super().__init__(f"{name} failed: {message} (code {status.code}, hip error {status.hip_error})")
@@ -119,8 +126,12 @@ SIGNATURES = {
                                                _I, _I, _I],
     "spar_hip_gradient_norm_summary": [ctypes.POINTER(NormSummary), _P, _U64, _I, _I],
     "spar_hip_launch_gradient_norm_summary": [_P, _P, _U64, _I, _I],
+    "spar_hip_launch_gradient_norm_summaries": [_P, _P, _U64P, _U64, _I, _I],
     "spar_hip_launch_scale_in_place": [_P, _U64, _I, _D, _I],
+    "spar_hip_launch_scale_in_place_batch": [_P, _U64P, _U64, _I, _D, _I],
     "spar_hip_launch_adamw": [_P, _P, _P, _P, _U64, _I, _D, _D, _D, _D, _D, _D, _D, _I],
+    "spar_hip_launch_adamw_batch": [ctypes.POINTER(AdamwTensor), _U64, _I, _D, _D, _D, _D, _D,
+                                    _I],
     "spar_hip_random_uniform": [_P, _U64, _I, _U64, _D, _D, _I],
     "spar_hip_random_normal": [_P, _U64, _I, _U64, _D, _D, _I],
 }

@@ -85,6 +85,51 @@ def test_adamw_bitexact(hip, dtype, hyper):
             assert_bitexact(gp, p, "parameter " + what)
 
 
+# Sizes around a vector, a tile (512 float32, 256 float64) and a segment
+# (4096, 2048), empty and unaligned tensors among them, one of 64 MiB (a launch
+# of its own), and more tensors than one launch takes (64 or 128).
+BATCH = [(0, 0), (1, 0), (3, 0), (255, 0), (256, 0), (257, 0), (511, 0), (513, 0), (5, 1),
+         (4097, 0), (0, 0), (1 << 18, 0), (70001, 1), (2049, 0),
+         (1 << 24, 0)] + [(7 * k + 1, 0) for k in range(130)]
+
+
+@pytest.mark.parametrize("dtype", [F32, F64])
+def test_batched_optimizer_calls(hip, dtype):
+    """The batched AdamW step, scaling and norm summaries give each tensor
+    what the oracle gives it alone, with its own bias corrections."""
+    rng = np.random.default_rng(107)
+    hyper = HYPER[0]
+    lr, b1, b2, eps, wd = hyper
+    arrays = [[(rng.standard_normal(n) * 0.1).astype(dtype) for _ in range(4)] for n, _ in BATCH]
+    for p, g, m, v in arrays:
+        np.abs(v, out=v)
+    placed = [[Placed(hip, a, offset) for a in four] for four, (_, offset) in zip(arrays, BATCH)]
+    counts = hip.u64_array([n for n, _ in BATCH])
+    gradients = (ctypes.c_void_p * len(BATCH))(*[four[1].ptr for four in placed])
+    size = ctypes.sizeof(hip.NormSummary)
+    out = hip.DeviceBuffer(size * len(BATCH))
+    hip.call("spar_hip_launch_gradient_norm_summaries", out.ptr, gradients, counts, len(BATCH),
+             hip.dtype_tag(dtype), 0)
+    raw = out.to_numpy(np.uint8, (len(BATCH), size))
+    tensors = (hip.AdamwTensor * len(BATCH))()
+    for k, ((n, _), four) in enumerate(zip(BATCH, placed)):
+        step = 1 + k % 3
+        tensors[k] = hip.AdamwTensor(four[0].ptr, four[1].ptr, four[2].ptr, four[3].ptr, n,
+                                     O.adamw_correction(b1, step), O.adamw_correction(b2, step))
+    hip.call("spar_hip_launch_adamw_batch", tensors, len(BATCH), hip.dtype_tag(dtype), lr, b1, b2,
+             eps, wd, 0)
+    hip.call("spar_hip_launch_scale_in_place_batch", gradients, counts, len(BATCH),
+             hip.dtype_tag(dtype), 0.37, 0)
+    for k, ((n, offset), (p, g, m, v)) in enumerate(zip(BATCH, arrays)):
+        what = f"tensor {k} n={n} offset={offset}"
+        check_summary(hip.NormSummary.from_buffer_copy(raw[k].tobytes()), g, what)
+        step = 1 + k % 3
+        scaled = (g.astype(F64) * 0.37).astype(dtype)
+        O.adamw(p, g, m, v, *hyper, O.adamw_correction(b1, step), O.adamw_correction(b2, step))
+        for got, want, name in zip(placed[k], (p, scaled, m, v), ("p", "g", "m", "v")):
+            assert_bitexact(got.numpy(), want, f"{name} of {what}")
+
+
 @pytest.mark.parametrize("dtype", [F32, F64])
 def test_adamw_special_values(hip, dtype):
     info = np.finfo(dtype)
