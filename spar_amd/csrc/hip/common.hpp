@@ -187,6 +187,16 @@ template <> struct Vec16<double> { using type = f64x2; static constexpr int widt
 template <> struct Vec16<int32_t> { using type = i32x4; static constexpr int width = 4; };
 template <> struct Vec16<int64_t> { using type = i64x2; static constexpr int width = 2; };
 
+// The same vectors at any element's address: gfx950 loads and stores 16 bytes
+// at element alignment in one instruction (the HSA ABI's unaligned access
+// mode), so rows of odd length keep wide accesses.
+typedef f32x4 f32x4_loose __attribute__((aligned(4)));
+typedef f64x2 f64x2_loose __attribute__((aligned(8)));
+
+template <typename T> struct Loose16;
+template <> struct Loose16<float> { using type = f32x4_loose; };
+template <> struct Loose16<double> { using type = f64x2_loose; };
+
 template <typename T>
 __device__ __forceinline__ T vec_get(const typename Vec16<T>::type& v, int i) {
   return v[i];
@@ -202,6 +212,12 @@ __device__ __forceinline__ void vec_set(typename Vec16<T>::type& v, int i, T x) 
 template <typename V>
 __device__ __forceinline__ V stream_load(const V* pointer) {
   return __builtin_nontemporal_load(pointer);
+}
+
+// 16 bytes from any element's address.
+template <typename T>
+__device__ __forceinline__ typename Vec16<T>::type loose_load(const T* pointer) {
+  return __builtin_nontemporal_load(reinterpret_cast<const typename Loose16<T>::type*>(pointer));
 }
 
 constexpr uint64_t kStreamStoreBytes = uint64_t{64} << 20;

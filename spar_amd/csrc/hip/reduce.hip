@@ -168,13 +168,21 @@ __device__ __forceinline__ T load_value(const T* a, const T* b, uint64_t offset)
   }
 }
 
-template <typename T, int NIN>
+// W elements from `offset` on; LOOSE: at any element's alignment.
+template <typename T, int NIN, bool LOOSE = false>
 __device__ __forceinline__ typename Vec16<T>::type load_vector(const T* a, const T* b,
                                                                uint64_t offset) {
   using V = typename Vec16<T>::type;
-  V va = stream_load(reinterpret_cast<const V*>(a + offset));
+  auto load = [](const T* at) {
+    if constexpr (LOOSE) {
+      return loose_load(at);
+    } else {
+      return stream_load(reinterpret_cast<const V*>(at));
+    }
+  };
+  V va = load(a + offset);
   if constexpr (NIN == 2) {
-    const V vb = stream_load(reinterpret_cast<const V*>(b + offset));
+    const V vb = load(b + offset);
 #pragma unroll
     for (int k = 0; k < Vec16<T>::width; ++k) {
       vec_set<T>(va, k, vec_get<T>(va, k) * vec_get<T>(vb, k));
@@ -475,6 +483,149 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// Combine of an accumulator over groups of L neighbouring lanes; every lane
+// gets its group's result.
+template <typename T, Kind K, int L>
+__device__ __forceinline__ Acc<T, K> group_reduce(Acc<T, K> acc) {
+#pragma unroll
+  for (int mask = L / 2; mask > 0; mask >>= 1) {
+    Acc<T, K> other;
+    if constexpr (K == Kind::Sum) {
+      other.value = __shfl_xor(acc.value, mask, kWave);
+    } else {
+      other.best.value = __shfl_xor(acc.best.value, mask, kWave);
+      other.best.index = __shfl_xor(acc.best.index, mask, kWave);
+    }
+    acc.merge(other);
+  }
+  return acc;
+}
+
+// Rows of kNarrowRow to kShortRow elements: L lanes per row (L a power of two
+// up to the wave, chosen so that a lane has one to four vectors), kThreads / L
+// rows per workgroup, combined by shuffles alone.  A workgroup per row left
+// most of its lanes without a load and spent two barriers on each row.  Loads
+// are 16 bytes at element alignment, so odd lengths take them too; the n % W
+// last elements go to the group's first lanes.  Sums of 2^24 float32 elements
+// in rows of 64 / 256 / 1000 took 288 / 76 / 23 us with a workgroup per row
+// and take 16.1 / 16.0 / 16.2 us; rows past 1024 give a workgroup's lanes a
+// vector each and stay with it.
+constexpr uint64_t kShortRow = 1024;
+
+template <typename T, Kind K, int NIN, int L>
+__global__ void __launch_bounds__(kThreads)
+    short_row_kernel(const T* a, const T* b, uint64_t rows, uint32_t n, RowMap map, Sink<T> sink) {
+  constexpr int W = Vec16<T>::width;
+  constexpr uint64_t kRows = kThreads / L;
+  const uint32_t lane = threadIdx.x % L;
+  const uint32_t body = n / W * W;
+  for (uint64_t first = static_cast<uint64_t>(blockIdx.x) * kRows; first < rows;
+       first += static_cast<uint64_t>(gridDim.x) * kRows) {
+    const uint64_t row = first + threadIdx.x / L;
+    ScanAcc<T, K> scan;
+    scan.init();
+    if (row < rows) {
+      const uint64_t base = row_offset(map, row);
+#pragma unroll 4
+      for (uint32_t i = lane * W; i < body; i += L * W) {
+        const auto v = load_vector<T, NIN, true>(a, b, base + i);
+#pragma unroll
+        for (int k = 0; k < W; ++k) scan.add(vec_get<T>(v, k), i + k);
+      }
+      const uint32_t last = body + lane;
+      if (last < n) scan.add(load_value<T, NIN>(a, b, base + last), last);
+    }
+    Acc<T, K> acc = group_reduce<T, K, L>(scan.finish(0));
+    if (row < rows && lane == 0) {
+      acc.seal(0);  // a row of only -inf: its first element
+      sink_write<T, K>(sink, row, acc, 0);
+    }
+  }
+}
+
+// The reduced axes of a plan with several of them, flattened (innermost
+// first); positions are 32-bit.
+struct ReducedWalk {
+  int rank;
+  FastDiv divisors[kMaxRank];
+  uint64_t strides[kMaxRank];
+
+  __device__ __forceinline__ uint64_t offset(uint32_t position) const {
+    uint64_t off = 0;
+    uint32_t rest = position;
+#pragma unroll
+    for (int k = 0; k < kMaxRank; ++k) {
+      if (k < rank) {
+        const uint32_t q = divisors[k].div(rest);
+        off += static_cast<uint64_t>(rest - q * divisors[k].divisor) * strides[k];
+        rest = q;
+      }
+    }
+    return off;
+  }
+};
+
+// Several reduced axes, the innermost contiguous (channel sums over [batch,
+// channel, pixel]): block b reduces positions [begin, begin + segment) of
+// output b / splits, decoding each load's position, four loads in flight.
+// VEC: the innermost reduced extent is a multiple of W, so a vector never
+// leaves its run.  A wave per output (the general kernel below) left 96
+// channels on 96 waves: the sums of [24, 96, 3136] over axes 0 and 2 took 772
+// us in float64 and 759 us in float32 there, and take 17.2 and 11.9 us here.
+template <typename T, Kind K, int NIN, bool VEC>
+__global__ void __launch_bounds__(kThreads)
+    run_kernel(const T* a, const T* b, uint64_t outputs, uint64_t count, uint64_t splits,
+               uint64_t segment, RowMap map, ReducedWalk walk, Sink<T> sink) {
+  constexpr uint64_t W = VEC ? Vec16<T>::width : 1;
+  constexpr int U = 4;
+  constexpr uint64_t step = static_cast<uint64_t>(kThreads) * W;
+  for (uint64_t block = blockIdx.x; block < outputs * splits; block += gridDim.x) {
+    const uint64_t output = block / splits;
+    const uint64_t begin = (block - output * splits) * segment;
+    const uint64_t end = begin + segment < count ? begin + segment : count;
+    const uint64_t base = row_offset(map, output);
+    ScanAcc<T, K> scan[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) scan[u].init();
+    // The accumulators' index is the position relative to `begin`.
+    auto add = [&](ScanAcc<T, K>& acc, const auto& v, uint64_t i) {
+      const uint32_t relative = static_cast<uint32_t>(i - begin);
+      if constexpr (VEC) {
+#pragma unroll
+        for (uint64_t k = 0; k < W; ++k) acc.add(vec_get<T>(v, k), relative + k);
+      } else {
+        acc.add(v, relative);
+      }
+    };
+    auto load = [&](uint64_t i) {
+      const uint64_t offset = base + walk.offset(static_cast<uint32_t>(i));
+      if constexpr (VEC) {
+        return load_vector<T, NIN, true>(a, b, offset);
+      } else {
+        return load_value<T, NIN>(a, b, offset);
+      }
+    };
+    uint64_t i = begin + threadIdx.x * W;
+    for (; i + (U - 1) * step < end; i += U * step) {
+      decltype(load(i)) v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = load(i + u * step);
+#pragma unroll
+      for (int u = 0; u < U; ++u) add(scan[u], v[u], i + u * step);
+    }
+    for (; i < end; i += step) add(scan[0], load(i), i);
+    Acc<T, K> acc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = scan[u].finish(static_cast<int64_t>(begin));
+    acc[0].merge(acc[1]);
+    acc[2].merge(acc[3]);
+    acc[0].merge(acc[2]);
+    Acc<T, K> total = block_reduce<T, K>(acc[0]);
+    if (begin < end) total.seal(static_cast<int64_t>(begin));
+    if (threadIdx.x == 0) sink_write<T, K>(sink, block, total, static_cast<int64_t>(begin));
+  }
+}
+
 // Second pass after row splits: one block per output reduces its `parts`
 // consecutive partials with a fixed tree.
 template <typename T, Kind K>
@@ -514,11 +665,13 @@ __global__ void __launch_bounds__(kThreads)
 // of the block's segment interleaved (wave w takes rows w, w+4, ...), so a
 // wave reads 1 KiB contiguous per row.  The four wave partials are combined
 // through LDS in wave order.  Block b covers column block cb, split s, outer o.
-template <typename T, Kind K, int NIN, bool VEC>
+// MULTI: several reduced axes, whose rows are found by decoding r (the same
+// for every lane of a wave).
+template <typename T, Kind K, int NIN, bool VEC, bool MULTI>
 __global__ void __launch_bounds__(kThreads)
     column_kernel(const T* a, const T* b, uint64_t outer, uint64_t n, uint64_t reduced_stride,
                   uint64_t inner, uint64_t column_blocks, uint64_t splits, uint64_t segment,
-                  RowMap map, Sink<T> sink) {
+                  RowMap map, ReducedWalk walk, Sink<T> sink) {
   constexpr int W = VEC ? Vec16<T>::width : 1;
   __shared__ Acc<T, K> lds[kWaves][kWave * W];
   const int wave = threadIdx.x / kWave;
@@ -537,13 +690,20 @@ __global__ void __launch_bounds__(kThreads)
     for (int k = 0; k < W; ++k) acc[k].init();
     if (column < inner) {
       const uint64_t base = row_offset(map, o) + column;
+      auto row = [&](uint64_t index) {
+        if constexpr (MULTI) {
+          return walk.offset(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(index)));
+        } else {
+          return index * reduced_stride;
+        }
+      };
       uint64_t r = begin + wave;
       if constexpr (VEC) {
         for (; r + 3 * kWaves < end; r += 4 * kWaves) {
           typename Vec16<T>::type v[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            v[u] = load_vector<T, NIN>(a, b, base + (r + u * kWaves) * reduced_stride);
+            v[u] = load_vector<T, NIN>(a, b, base + row(r + u * kWaves));
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
@@ -554,13 +714,13 @@ __global__ void __launch_bounds__(kThreads)
           }
         }
         for (; r < end; r += kWaves) {
-          const auto v = load_vector<T, NIN>(a, b, base + r * reduced_stride);
+          const auto v = load_vector<T, NIN>(a, b, base + row(r));
 #pragma unroll
           for (int k = 0; k < W; ++k) acc[k].add(vec_get<T>(v, k), static_cast<int64_t>(r));
         }
       } else {
         for (; r < end; r += kWaves) {
-          acc[0].add(load_value<T, NIN>(a, b, base + r * reduced_stride), static_cast<int64_t>(r));
+          acc[0].add(load_value<T, NIN>(a, b, base + row(r)), static_cast<int64_t>(r));
         }
       }
     }
@@ -1114,8 +1274,20 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
   };
 
   const bool row_case = plan.red_rank == 1 && plan.red_strides[0] == 1;
-  const bool column_case = !row_case && plan.red_rank == 1 && plan.kept_rank >= 1 &&
-                           plan.kept_strides[plan.kept_rank - 1] == 1;
+  // Several reduced axes are walked by position where that fits 32 bits.
+  const bool multi = plan.red_rank > 1 && plan.reduced <= kIndex32Limit;
+  const bool run_case = multi && plan.red_strides[plan.red_rank - 1] == 1;
+  const bool column_case = !row_case && !run_case && (plan.red_rank == 1 || multi) &&
+                           plan.kept_rank >= 1 && plan.kept_strides[plan.kept_rank - 1] == 1;
+  ReducedWalk walk{};
+  if (multi) {
+    walk.rank = plan.red_rank;
+    for (int k = 0; k < plan.red_rank; ++k) {
+      const int axis = plan.red_rank - 1 - k;
+      walk.divisors[k].init(static_cast<uint32_t>(plan.red_extents[axis]));
+      walk.strides[k] = plan.red_strides[axis];
+    }
+  }
 
   if (plan.red_rank == 0) {
     // Nothing is reduced (all reduced extents are 1): a reduction of one
@@ -1134,6 +1306,28 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     if (n <= kNarrowRow) {
       narrow_row_kernel<T, K, NIN><<<grid_for((rows + kThreads - 1) / kThreads), kThreads, 0,
                                      guard.stream>>>(a, b, rows, n, 1, map, final_sink());
+      return hipSuccess;
+    }
+    if (n <= kShortRow) {
+      // lanes per row: about two vectors each, all of a wave from 256 elements
+      // (float32) on
+      auto launch = [&](auto lanes) {
+        constexpr int L = decltype(lanes)::value;
+        constexpr uint64_t kRows = kThreads / L;
+        short_row_kernel<T, K, NIN, L><<<grid_for((rows + kRows - 1) / kRows), kThreads, 0,
+                                         guard.stream>>>(a, b, rows, static_cast<uint32_t>(n), map,
+                                                         final_sink());
+      };
+      const uint64_t vectors = n / W;
+      if (vectors <= 16) {
+        launch(std::integral_constant<int, 8>{});
+      } else if (vectors <= 32) {
+        launch(std::integral_constant<int, 16>{});
+      } else if (vectors <= 64) {
+        launch(std::integral_constant<int, 32>{});
+      } else {
+        launch(std::integral_constant<int, 64>{});
+      }
       return hipSuccess;
     }
     bool vec = n % W == 0 && plan.offset % W == 0 && aligned16(a) && (NIN == 1 || aligned16(b));
@@ -1188,14 +1382,48 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     });
   }
 
+  if (run_case) {
+    const uint64_t outputs = plan.outputs;
+    const uint64_t count = plan.reduced;
+    const RowMap map = make_row_map(plan, plan.kept_rank);
+    const bool vec = plan.red_extents[plan.red_rank - 1] % W == 0;
+    const uint64_t width = vec ? W : 1;
+    const uint64_t min_segment = static_cast<uint64_t>(kThreads) * width * 8;
+    uint64_t splits = 1;
+    if (outputs < target_blocks && count >= 2 * min_segment) {
+      splits = (target_blocks + outputs - 1) / outputs;
+      if (splits > count / min_segment) splits = count / min_segment;
+    }
+    const uint64_t segment = ((count + splits - 1) / splits + width - 1) / width * width;
+    splits = (count + segment - 1) / segment;
+    auto launch = [&](const Sink<T>& s) {
+      auto kernel = vec ? run_kernel<T, K, NIN, true> : run_kernel<T, K, NIN, false>;
+      kernel<<<grid_for(outputs * splits), kThreads, 0, guard.stream>>>(a, b, outputs, count,
+                                                                        splits, segment, map, walk,
+                                                                        s);
+    };
+    if (splits == 1) {
+      launch(final_sink());
+      return hipSuccess;
+    }
+    return with_partials(outputs * splits, [&](const Sink<T>& partial) {
+      launch(partial);
+      combine_rows_kernel<T, K><<<grid_for(outputs), kThreads, 0, guard.stream>>>(
+          partial.values, partial.partial_indices, outputs, splits, segment, final_sink());
+    });
+  }
+
   if (column_case) {
     const uint64_t inner = plan.kept_extents[plan.kept_rank - 1];
     const uint64_t outer = plan.outputs / inner;
-    const uint64_t n = plan.red_extents[0];
-    const uint64_t reduced_stride = plan.red_strides[0];
+    const uint64_t n = plan.reduced;
+    const uint64_t reduced_stride = plan.red_strides[0];  // of the one reduced axis
     const RowMap map = make_row_map(plan, plan.kept_rank - 1);
-    bool vec = inner % W == 0 && plan.offset % W == 0 && reduced_stride % W == 0 &&
-               aligned16(a) && (NIN == 1 || aligned16(b));
+    bool vec = inner % W == 0 && plan.offset % W == 0 && aligned16(a) &&
+               (NIN == 1 || aligned16(b));
+    for (int k = 0; k < plan.red_rank; ++k) {
+      if (plan.red_strides[k] % W != 0) vec = false;
+    }
     for (int k = 0; k < plan.kept_rank - 1; ++k) {
       if (plan.kept_strides[k] % W != 0) vec = false;
     }
@@ -1206,7 +1434,7 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     if constexpr (K == Kind::Max) {
       constexpr uint64_t kStripColumns = static_cast<uint64_t>(kStripGroups) * W;
       const uint64_t strips = outer * ((inner + kStripColumns - 1) / kStripColumns);
-      if (vec && n < kMaxScanRange && n >= static_cast<uint64_t>(kStripRows) * 8 &&
+      if (vec && !multi && n < kMaxScanRange && n >= static_cast<uint64_t>(kStripRows) * 8 &&
           strips >= static_cast<uint64_t>(cus)) {
         column_strip_kernel<T, K, NIN, 8><<<grid_for(strips), kThreads, 0, guard.stream>>>(
             a, b, outer, n, reduced_stride, inner, map, final_sink());
@@ -1218,31 +1446,60 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     // split; other wide rows 1 group per lane, 4 rows in flight, 2 blocks per
     // CU and >= 64 rows per split.  Narrow rows: waves interleave rows (8
     // blocks per CU, >= 16 rows per wave).
-    const bool wide = vec && inner / W >= static_cast<uint64_t>(kWaves) * kWave;
-    const bool quad = wide && (inner / W) % (static_cast<uint64_t>(kThreads) * 4) == 0;
-    const uint64_t columns_per_block = static_cast<uint64_t>(kWave) * (vec ? W : 1) *
-                                       (wide ? kWaves : 1) * (quad ? 4 : 1);
-    const uint64_t column_blocks = (inner + columns_per_block - 1) / columns_per_block;
-    const uint64_t base_blocks = outer * column_blocks;
-    uint64_t splits = 1;
-    const uint64_t min_rows = quad ? 16 : wide ? 64 : 16 * kWaves;
-    const uint64_t wanted_blocks = static_cast<uint64_t>(cus) * (quad ? 1 : wide ? 2 : 8);
-    if (base_blocks < wanted_blocks && n >= 2 * min_rows) {
-      splits = (wanted_blocks + base_blocks - 1) / base_blocks;
-      if (splits > n / min_rows) splits = n / min_rows;
-      if (splits < 1) splits = 1;
+    struct Shape {
+      bool wide;
+      bool quad;
+      uint64_t column_blocks;
+      uint64_t splits;
+    };
+    auto shape_of = [&](bool wide) {
+      const bool quad = wide && (inner / W) % (static_cast<uint64_t>(kThreads) * 4) == 0;
+      const uint64_t columns_per_block = static_cast<uint64_t>(kWave) * (vec ? W : 1) *
+                                         (wide ? kWaves : 1) * (quad ? 4 : 1);
+      const uint64_t column_blocks = (inner + columns_per_block - 1) / columns_per_block;
+      const uint64_t base_blocks = outer * column_blocks;
+      uint64_t splits = 1;
+      const uint64_t min_rows = quad ? 16 : wide ? 64 : 16 * kWaves;
+      const uint64_t wanted_blocks = static_cast<uint64_t>(cus) * (quad ? 1 : wide ? 2 : 8);
+      if (base_blocks < wanted_blocks && n >= 2 * min_rows) {
+        splits = (wanted_blocks + base_blocks - 1) / base_blocks;
+        if (splits > n / min_rows) splits = n / min_rows;
+        if (splits < 1) splits = 1;
+      }
+      return Shape{wide, quad, column_blocks, splits};
+    };
+    const uint64_t slot_bytes = sizeof(T) + (K == Kind::Max ? sizeof(uint32_t) : 0);
+    const uint64_t most_splits = workspace.fixed == nullptr
+                                     ? UINT64_MAX
+                                     : (workspace.capacity - 256) / slot_bytes / (outer * inner);
+    Shape shape = shape_of(vec && !multi && inner / W >= static_cast<uint64_t>(kWaves) * kWave);
+    // Rows that are wide but too few to split well, in waves that do not fill
+    // the chip, are interleaved as well, over four times the waves: the sum of
+    // [24, 96, 3136] float32 over axis 1 took 17.1 us with 168 workgroups of
+    // 96-row waves and takes 8.0 us, of [32, 32, 8192] 13.8 and 8.1 us; from
+    // 128 rows or two workgroups of waves per CU on the wide scan is ahead.
+    // (A request that the fixed workspace refused stays refused.)
+    const uint64_t wide_blocks = outer * ((inner / W + kThreads - 1) / kThreads);
+    if (shape.wide && n < 128 && wide_blocks < static_cast<uint64_t>(cus) * 2 &&
+        shape.splits <= most_splits) {
+      shape = shape_of(false);
     }
-    const uint64_t range_splits = (n + kMaxScanRange / 2 - 1) / (kMaxScanRange / 2);
+    // several reduced axes never asked for a workspace: one split needs none
+    if (multi && shape.splits > most_splits) shape.splits = most_splits < 1 ? 1 : most_splits;
+    const uint64_t column_blocks = shape.column_blocks;
+    uint64_t splits = shape.splits;
+    const uint64_t range_splits =
+        multi ? 1 : (n + kMaxScanRange / 2 - 1) / (kMaxScanRange / 2);
     if (splits < range_splits) splits = range_splits;
     const uint64_t segment = (n + splits - 1) / splits;
     splits = (n + segment - 1) / segment;
     // A max without argmax over wide rows scans and combines values only.
-    const bool value_only = K == Kind::Max && operation == SPAR_HIP_MAX && wide;
+    const bool value_only = K == Kind::Max && operation == SPAR_HIP_MAX && shape.wide;
     auto launch = [&](const Sink<T>& s) {
       const uint32_t grid = grid_for(outer * splits * column_blocks);
       auto launch_wide = [&](auto index) {
         constexpr bool INDEX = decltype(index)::value;
-        if (quad) {
+        if (shape.quad) {
           column_wide_kernel<T, K, NIN, 4, 2, INDEX><<<grid, kThreads, 0, guard.stream>>>(
               a, b, outer, n, reduced_stride, inner, column_blocks, splits, segment, map, s);
         } else {
@@ -1250,7 +1507,7 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
               a, b, outer, n, reduced_stride, inner, column_blocks, splits, segment, map, s);
         }
       };
-      if (wide) {
+      if (shape.wide) {
         if constexpr (K == Kind::Max) {
           if (value_only) {
             launch_wide(std::false_type{});
@@ -1258,12 +1515,13 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
           }
         }
         launch_wide(std::true_type{});
-      } else if (vec) {
-        column_kernel<T, K, NIN, true><<<grid, kThreads, 0, guard.stream>>>(
-            a, b, outer, n, reduced_stride, inner, column_blocks, splits, segment, map, s);
       } else {
-        column_kernel<T, K, NIN, false><<<grid, kThreads, 0, guard.stream>>>(
-            a, b, outer, n, reduced_stride, inner, column_blocks, splits, segment, map, s);
+        auto kernel = multi ? (vec ? column_kernel<T, K, NIN, true, true>
+                                   : column_kernel<T, K, NIN, false, true>)
+                            : (vec ? column_kernel<T, K, NIN, true, false>
+                                   : column_kernel<T, K, NIN, false, false>);
+        kernel<<<grid, kThreads, 0, guard.stream>>>(a, b, outer, n, reduced_stride, inner,
+                                                    column_blocks, splits, segment, map, walk, s);
       }
     };
     if (splits == 1) {

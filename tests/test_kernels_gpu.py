@@ -620,6 +620,60 @@ def test_short_row_reductions_exact(hip, dtype, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [33, 63, 64, 65, 129, 130, 255, 257, 511, 513, 1023, 1024, 1025])
+def test_short_rows_by_lane_groups(hip, dtype, n):
+    """Rows of 33 to 1024 elements take a group of 8 to 64 lanes each (1025:
+    the workgroup kernel), at element alignment: every row start of the block
+    is misaligned for 16 bytes, and 301 rows leave a last workgroup partly
+    empty.  NaNs, ties and rows of only -inf keep the first-occurrence rule."""
+    base = inputs(n, 301 * (n + 3), dtype, with_specials=False).reshape(301, n + 3)
+    base[5, :] = -np.inf
+    check_axis(hip, base, base[:, 1:1 + n], [1], dtype, f"lane groups n={n}")
+    spiked = np.round(base)
+    spiked[7, [n // 2, n - 1]] = np.nan
+    mx, am = ref.axis_max(spiked[:, 1:1 + n], [1])
+    for op, want in (("max", mx), ("argmax", am)):
+        got = axis_reduce(hip, spiked, spiked[:, 1:1 + n], [1], op, dtype)
+        assert_bitexact(got, want, f"lane groups {op} with ties and NaNs n={n}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape,order,axes", [
+    ((5, 7, 9), (0, 1, 2), [0, 2]),               # runs of odd length, no split
+    ((40, 3, 1028), (0, 1, 2), [0, 2]),           # vector runs, split outputs
+    ((40, 2, 1031), (0, 1, 2), [0, 2]),           # odd runs, split
+    ((6, 5, 4, 33), (0, 1, 2, 3), [0, 1, 3]),     # two outer reduced axes
+    ((3, 4, 5, 6, 7, 8), (0, 1, 2, 3, 4, 5), [1, 3, 5]),
+    ((9, 31, 5, 36), (0, 1, 2, 3), [0, 2]),       # columns, two reduced axes
+    ((9, 31, 5, 37), (0, 1, 2, 3), [0, 2]),       # columns of odd width
+    ((4, 8, 65, 264), (2, 0, 1, 3), [0, 1]),      # permuted, split over rows
+    ((13, 6, 10, 4), (3, 1, 2, 0), [0, 1, 2]),    # nothing contiguous kept
+])
+def test_several_reduced_axes(hip, dtype, shape, order, axes):
+    """Several reduced axes that do not merge: the innermost contiguous (runs)
+    or the kept axis contiguous (columns), from offset views."""
+    total = int(np.prod(shape))
+    base = inputs(61, total + 3, dtype, with_specials=False)
+    view = base[3:].reshape(shape).transpose(order)
+    check_axis(hip, base, view, axes, dtype, f"{shape} {order} {axes}")
+    spiked = np.round(base * 2)
+    spiked[[total // 3, total // 2, total]] = np.nan
+    view = spiked[3:].reshape(shape).transpose(order)
+    mx, am = ref.axis_max(view, axes)
+    for op, want in (("max", mx), ("argmax", am)):
+        assert_bitexact(axis_reduce(hip, spiked, view, axes, op, dtype), want,
+                        f"{op} with ties and NaNs {shape} {order} {axes}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(24, 96, 784), (3, 127, 3136), (2, 128, 3136), (5, 31, 4096)])
+def test_few_wide_rows(hip, dtype, shape):
+    """Fewer than 128 wide rows on too few waves take the interleaved scan."""
+    base = inputs(62, int(np.prod(shape)), dtype, with_specials=False).reshape(shape)
+    check_axis(hip, base, base, [1], dtype, f"few wide rows {shape}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape,axes", [((300, 2048), [0]), ((3, 200, 1100), [1]),
                                         ((2, 70, 4096), [0, 1]), ((5000, 1024), [0])])
 def test_column_reductions_wide_rows(hip, dtype, shape, axes):

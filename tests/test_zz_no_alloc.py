@@ -108,6 +108,28 @@ def test_no_alloc_layouts(hip, op):
     assert_bitexact(got, want, f"{op} [257,1000] axis 0")
 
 
+def test_no_alloc_keeps_several_axes_within_the_workspace(hip):
+    # Column sums over two axes that do not merge never needed a workspace:
+    # [256, 2, 4, 1024, 128] over axes 0 and 2 has 262,144 float64 outputs,
+    # whose splits would take 4 MiB (argmax 3 MiB) each, so they are capped to
+    # what fits.
+    shape = [256, 2, 4, 1024, 128]
+    x = normal(hip, int(np.prod(shape)), 36, np.float32)
+    strides = [2 * 4 * 1024 * 128, 4 * 1024 * 128, 1024 * 128, 128, 1]
+    say(f"no_alloc MAX, ARGMAX, SUM {shape} axes 0, 2")
+    host = x.to_numpy(np.float32, shape)
+    for op in ("MAX", "ARGMAX"):
+        want, got = run_both(hip, x, shape, strides, 0, 5, np.float32, getattr(hip, op))
+        assert_bitexact(got, want, f"{op} {shape}")
+        if op == "MAX":
+            assert_bitexact(got, host.max(axis=(0, 2)).reshape(-1), "MAX of numpy")
+    # sums: the splits, and so the order, may differ between the entry points
+    want, got = run_both(hip, x, shape, strides, 0, 5, np.float32, hip.SUM)
+    exact = host.sum(axis=(0, 2), dtype=np.float64).reshape(-1)
+    bound = 1024 * 2.0 ** -24 * np.abs(host).sum(axis=(0, 2), dtype=np.float64).reshape(-1)
+    assert (np.abs(got - exact) <= bound).all() and (np.abs(want - exact) <= bound).all()
+
+
 def test_no_alloc_refuses_plans_beyond_the_workspace(hip):
     # float32 argmax over axis 0 of [32, (cus - 1) * 4096]: cus - 1 column
     # blocks of 4096 columns, one short of one block per CU, so the planner
