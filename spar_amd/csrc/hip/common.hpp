@@ -247,6 +247,13 @@ __device__ __forceinline__ void store_vector(V* pointer, V value) {
   }
 }
 
+// 16 bytes to any element's address.
+template <bool NT, typename T>
+__device__ __forceinline__ void loose_store(T* pointer, typename Vec16<T>::type value) {
+  store_vector<NT>(reinterpret_cast<typename Loose16<T>::type*>(pointer),
+                   static_cast<typename Loose16<T>::type>(value));
+}
+
 template <bool NT, typename V>
 __device__ __forceinline__ V load_vector_policy(const V* pointer) {
   if constexpr (NT) {

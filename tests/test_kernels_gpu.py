@@ -1168,6 +1168,59 @@ def test_softmax_rows_beyond_one_grid(hip):
     assert np.all(np.isnan(got[-1]))
 
 
+# [outer, axis, inner] at the edges of the slice kernels' shapes: 16-byte units
+# (inner from 32 on, also not a multiple of the vector) and single slices, rows
+# per lane group full, partial and one past, few and many workgroups, looped.
+SLICE_SHAPES = [(3, 1, 40), (2, 16, 32), (3, 17, 33), (2, 64, 47), (2, 65, 64), (1, 256, 130),
+                (2, 257, 66), (1, 512, 100), (300, 513, 36), (1, 1025, 35), (1, 2048, 33),
+                (1, 2049, 34), (200, 300, 64), (130, 1100, 40), (5, 16, 2), (7, 17, 31),
+                (3, 64, 5), (2, 65, 7), (2, 257, 3), (1, 1024, 30), (1, 1025, 2), (1, 2100, 9),
+                (2000, 300, 3), (3000, 520, 2), (2500, 1030, 3)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", SLICE_SHAPES)
+def test_softmax_slices(hip, dtype, shape):
+    """Softmax and log-softmax along a middle axis, forward and backward,
+    with undefined slices (NaN, +inf, all -inf) beside defined ones."""
+    outer, axis, inner = shape
+    x = (inputs(63, int(np.prod(shape)), dtype, with_specials=False) * dtype(1.5)).reshape(shape)
+    x[0, axis // 2, 0] = np.nan
+    x[-1, :, -1] = -np.inf
+    x[-1, 0, inner // 2] = np.inf
+    x[-1, axis - 1, inner // 2] = np.inf
+    x[0, 0, 1] = -np.inf if axis > 1 else 0.0
+    g = inputs(64, x.size, dtype, with_specials=False).reshape(shape)
+    for log in (False, True):
+        want, und_ref = (ref.log_softmax(x, 1) if log else ref.softmax_axis(x, 1))
+        got, und = softmax_device(hip, x, outer, axis, inner, log, dtype)
+        flags = und_ref.astype(np.int32)
+        assert np.array_equal(und, flags)
+        defined = np.broadcast_to((flags.reshape(outer, 1, inner) == 0), shape)
+        special = (~defined) | np.isinf(want)
+        assert_ulp(got[special], want[special], 2, f"undefined slices {shape} log={log}")
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        finite_got, finite_want = (np.where(special, 0, a).astype(dtype) for a in (got, want))
+        check = log_softmax_tolerance_check if log else softmax_tolerance_check
+        check(finite_got, finite_want, axis, dtype, f"slices {shape} log={log}")
+        out = out_buf(hip, shape, dtype)
+        hip.call("spar_hip_launch_probability_backward", out.ptr, dev(hip, g).ptr,
+                 dev(hip, want).ptr, dev(hip, flags).ptr, outer, axis, inner, tag(dtype),
+                 int(log), 0)
+        back = out.to_numpy(dtype, shape).astype(np.float64)
+        assert np.array_equal(np.isnan(back), ~defined)
+        # against float64, with the bound of an axis-long sum
+        y = np.where(defined, want, 0).astype(np.float64)
+        gd = g.astype(np.float64)
+        p = np.exp(y) if log else y
+        s = gd.sum(1, keepdims=True) if log else (gd * y).sum(1, keepdims=True)
+        exact = gd - p * s if log else y * (gd - s)
+        magnitude = (np.abs(gd) if log else np.abs(gd * y)).sum(1, keepdims=True)
+        u = np.finfo(dtype).eps
+        bound = (axis + 8) * u * p * magnitude + 4 * u * (np.abs(gd) + np.abs(exact))
+        assert (np.abs(back - exact) <= bound)[defined].all(), f"backward {shape} log={log}"
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape,axis", [((6, 50, 33), 1), ((40, 9), 0), ((3, 4, 5, 6), 2)])
 def test_softmax_inner_axis(hip, dtype, shape, axis):
