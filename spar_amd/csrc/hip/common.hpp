@@ -214,10 +214,11 @@ __device__ __forceinline__ V stream_load(const V* pointer) {
   return __builtin_nontemporal_load(pointer);
 }
 
-// 16 bytes from any element's address.
+// 16 bytes from any element's address: a cached load, since a misaligned
+// wave shares its first and last lines with its neighbours.
 template <typename T>
 __device__ __forceinline__ typename Vec16<T>::type loose_load(const T* pointer) {
-  return __builtin_nontemporal_load(reinterpret_cast<const typename Loose16<T>::type*>(pointer));
+  return *reinterpret_cast<const typename Loose16<T>::type*>(pointer);
 }
 
 constexpr uint64_t kStreamStoreBytes = uint64_t{64} << 20;

@@ -507,9 +507,9 @@ __device__ __forceinline__ Acc<T, K> group_reduce(Acc<T, K> acc) {
 // most of its lanes without a load and spent two barriers on each row.  Loads
 // are 16 bytes at element alignment, so odd lengths take them too; the n % W
 // last elements go to the group's first lanes.  Sums of 2^24 float32 elements
-// in rows of 64 / 256 / 1000 took 288 / 76 / 23 us with a workgroup per row
-// and take 16.1 / 16.0 / 16.2 us; rows past 1024 give a workgroup's lanes a
-// vector each and stay with it.
+// in rows of 49 / 64 / 256 / 1000 took 331 / 286 / 75 / 23.1 us with a
+// workgroup per row and take 17.1 / 13.6 / 13.8 / 13.6 us; rows past 1024 give
+// a workgroup's lanes a vector each and stay with it.
 constexpr uint64_t kShortRow = 1024;
 
 template <typename T, Kind K, int NIN, int L>
@@ -571,7 +571,7 @@ struct ReducedWalk {
 // VEC: the innermost reduced extent is a multiple of W, so a vector never
 // leaves its run.  A wave per output (the general kernel below) left 96
 // channels on 96 waves: the sums of [24, 96, 3136] over axes 0 and 2 took 772
-// us in float64 and 759 us in float32 there, and take 17.2 and 11.9 us here.
+// us in float64 and 759 us in float32 there, and take 17.0 and 11.8 us here.
 template <typename T, Kind K, int NIN, bool VEC>
 __global__ void __launch_bounds__(kThreads)
     run_kernel(const T* a, const T* b, uint64_t outputs, uint64_t count, uint64_t splits,

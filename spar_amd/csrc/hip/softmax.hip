@@ -19,6 +19,8 @@
 // workgroup by rows and by neighbouring slices.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "ops.hpp"
 
@@ -81,10 +83,11 @@ __device__ __forceinline__ void stats_merge(SliceStats<T>& s, const SliceStats<T
   stats_max(s, o.value, o.index);
 }
 
-template <typename T>
-__device__ __forceinline__ SliceStats<T> wave_stats(SliceStats<T> s) {
+// Merged over groups of L neighbouring lanes.
+template <typename T, int L>
+__device__ __forceinline__ SliceStats<T> lane_stats(SliceStats<T> s) {
 #pragma unroll
-  for (int mask = kWave / 2; mask > 0; mask >>= 1) {
+  for (int mask = L / 2; mask > 0; mask >>= 1) {
     SliceStats<T> o;
     o.value = __shfl_xor(s.value, mask, kWave);
     o.index = __shfl_xor(s.index, mask, kWave);
@@ -101,7 +104,7 @@ template <typename T, int THREADS, bool GUARD = true>
 __device__ __forceinline__ SliceStats<T> block_stats(SliceStats<T> s) {
   constexpr int kWavesPerBlock = THREADS / kWave;
   __shared__ SliceStats<T> lds[kWavesPerBlock];
-  s = wave_stats(s);
+  s = lane_stats<T, kWave>(s);
   if constexpr (GUARD) exchange_barrier();
   if (threadIdx.x % kWave == 0) lds[threadIdx.x / kWave] = s;
   exchange_barrier();
@@ -177,115 +180,107 @@ __device__ __forceinline__ bool slice_undefined(const SliceStats<T>& s) {
   return s.nan != 0 || s.value == -positive_infinity<T>() || s.positive_infinities != 0;
 }
 
-// Element j of a thread's register array maps to column col(t, j):
-// VEC: 16-byte groups interleaved across lanes; scalar: lanes interleaved.
-// Register rows hold at most 32768 elements, so columns are 32-bit and a
-// row access is a uniform row base plus a 32-bit lane offset.
-template <typename T, int THREADS, bool VEC>
+// A row's L lanes (a power of two: part of a wave, a wave or a workgroup) hold
+// it in registers: slot j of lane l is column (j / W * L + l) * W + j % W, 16
+// bytes interleaved across lanes.  Register rows hold at most 65536 elements,
+// so columns are 32-bit and a row access is a uniform row base plus a 32-bit
+// lane offset.
+template <typename T, int L>
 __device__ __forceinline__ uint32_t column_of(int j) {
-  if constexpr (VEC) {
-    constexpr int W = Vec16<T>::width;
-    return (static_cast<uint32_t>(j / W) * THREADS + threadIdx.x) * W + (j % W);
-  } else {
-    return static_cast<uint32_t>(j) * THREADS + threadIdx.x;
-  }
+  constexpr int W = Vec16<T>::width;
+  return (static_cast<uint32_t>(j / W) * L + threadIdx.x % L) * W + (j % W);
 }
 
 // Columns grow with the register slot j, so the slots of a lane that hold
-// columns < n are a prefix j < live_slots(n) (whole 16-byte groups for VEC,
-// where n is a multiple of the vector width).  One 32-bit bound per lane
-// replaces a 64-bit column compare per slot.
-template <typename T, int THREADS, int E, bool VEC>
+// whole 16-byte groups of columns < n are a prefix j < live_slots(n).  One
+// 32-bit bound per lane replaces a 64-bit column compare per slot.
+template <typename T, int L, int E>
 __device__ __forceinline__ int live_slots(uint64_t n) {
-  constexpr int W = VEC ? Vec16<T>::width : 1;
-  const int units = static_cast<int>(n / W);  // n <= THREADS * E
-  const int lane = static_cast<int>(threadIdx.x);
-  return units > lane ? ((units - lane + THREADS - 1) / THREADS) * W : 0;
+  constexpr int W = Vec16<T>::width;
+  const int units = static_cast<int>(n / W);  // n <= L * E
+  const int lane = static_cast<int>(threadIdx.x % L);
+  return units > lane ? ((units - lane + L - 1) / L) * W : 0;
+}
+
+// How a row kernel's rows lie: kWhole: aligned and exactly filling the
+// registers; kGroups: aligned and a whole number of 16-byte groups; kOdd: any
+// length at any element's alignment, moved 16 bytes at a time, with the n % W
+// last elements in one more slot of the first lanes.  Odd rows take ordinary
+// stores: neighbouring lanes and rows share their cache lines, and
+// non-temporal ones took 71 us where these take 49 us on [2048, 16385] float32
+// softmax.
+constexpr int kWhole = 0;
+constexpr int kGroups = 1;
+constexpr int kOdd = 2;
+
+template <int E, int LAYOUT>
+constexpr int kRowSlots = LAYOUT == kOdd ? E + 1 : E;
+
+// Column of a lane's slot; that of the last slot of an odd row is n or more
+// where it holds nothing.
+template <typename T, int L, int E>
+__device__ __forceinline__ uint32_t slot_column(int j, uint64_t n) {
+  constexpr uint32_t W = Vec16<T>::width;
+  if (j < E) return column_of<T, L>(j);
+  return static_cast<uint32_t>(n) / W * W + threadIdx.x % L;
 }
 
 // Loads a row into registers; slots past the row hold `pad`.
-template <typename T, int THREADS, int E, bool VEC, bool FULL>
-__device__ __forceinline__ void load_row(T (&x)[E], const T* row, int live, T pad) {
-  if constexpr (VEC) {
-    using V = typename Vec16<T>::type;
-    constexpr int W = Vec16<T>::width;
+template <typename T, int L, int E, int LAYOUT, int N>
+__device__ __forceinline__ void load_row(T (&x)[N], const T* row, uint64_t n, int live, T pad) {
+  static_assert(N == kRowSlots<E, LAYOUT>);
+  using V = typename Vec16<T>::type;
+  constexpr int W = Vec16<T>::width;
 #pragma unroll
-    for (int v = 0; v < E / W; ++v) {
-      if (FULL || v * W < live) {
-        const V value = stream_load(reinterpret_cast<const V*>(row + column_of<T, THREADS, true>(v * W)));
-#pragma unroll
-        for (int k = 0; k < W; ++k) x[v * W + k] = vec_get<T>(value, k);
+  for (int v = 0; v < E / W; ++v) {
+    if (LAYOUT == kWhole || v * W < live) {
+      const T* at = row + column_of<T, L>(v * W);
+      V value;
+      if constexpr (LAYOUT == kOdd) {
+        value = loose_load(at);
       } else {
-#pragma unroll
-        for (int k = 0; k < W; ++k) x[v * W + k] = pad;
+        value = stream_load(reinterpret_cast<const V*>(at));
       }
-    }
-  } else {
 #pragma unroll
-    for (int j = 0; j < E; ++j) x[j] = FULL || j < live ? row[column_of<T, THREADS, false>(j)] : pad;
+      for (int k = 0; k < W; ++k) x[v * W + k] = vec_get<T>(value, k);
+    } else {
+#pragma unroll
+      for (int k = 0; k < W; ++k) x[v * W + k] = pad;
+    }
+  }
+  if constexpr (LAYOUT == kOdd) {
+    const uint32_t column = slot_column<T, L, E>(E, n);
+    x[E] = column < n ? row[column] : pad;
   }
 }
 
 // NT: non-temporal stores (outputs of 64 MiB or more).
-template <typename T, int THREADS, int E, bool VEC, bool FULL, bool NT>
-__device__ __forceinline__ void store_row(T* row, const T (&y)[E], int live) {
-  if constexpr (VEC) {
-    using V = typename Vec16<T>::type;
-    constexpr int W = Vec16<T>::width;
+template <typename T, int L, int E, int LAYOUT, bool NT, int N>
+__device__ __forceinline__ void store_row(T* row, const T (&y)[N], uint64_t n, int live) {
+  static_assert(N == kRowSlots<E, LAYOUT>);
+  using V = typename Vec16<T>::type;
+  constexpr int W = Vec16<T>::width;
 #pragma unroll
-    for (int v = 0; v < E / W; ++v) {
-      if (FULL || v * W < live) {
-        const uint32_t col = column_of<T, THREADS, true>(v * W);
-        V value;
+  for (int v = 0; v < E / W; ++v) {
+    if (LAYOUT == kWhole || v * W < live) {
+      T* at = row + column_of<T, L>(v * W);
+      V value;
 #pragma unroll
-        for (int k = 0; k < W; ++k) vec_set<T>(value, k, y[v * W + k]);
-        store_vector<NT>(reinterpret_cast<V*>(row + col), value);
+      for (int k = 0; k < W; ++k) vec_set<T>(value, k, y[v * W + k]);
+      if constexpr (LAYOUT == kOdd) {
+        loose_store<false>(at, value);
+      } else {
+        store_vector<NT>(reinterpret_cast<V*>(at), value);
       }
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      if (FULL || j < live) row[column_of<T, THREADS, false>(j)] = y[j];
-    }
+  }
+  if constexpr (LAYOUT == kOdd) {
+    const uint32_t column = slot_column<T, L, E>(E, n);
+    if (column < n) row[column] = y[E];
   }
 }
 
 // ----------------------------------------------------- register-row kernels
-
-// Block-wide first-occurrence maximum of (value, column) pairs: the larger
-// value wins, equal values (including -0 and +0) keep the smaller column.
-// NaN never enters (a lane only takes an element that compares larger).
-template <typename T, int THREADS, bool GUARD = true>
-__device__ __forceinline__ T block_max_first(T value, int32_t index) {
-  constexpr int kWavesPerBlock = THREADS / kWave;
-  __shared__ T lds_value[kWavesPerBlock];
-  __shared__ int32_t lds_index[kWavesPerBlock];
-#pragma unroll
-  for (int mask = kWave / 2; mask > 0; mask >>= 1) {
-    const T other = __shfl_xor(value, mask, kWave);
-    const int32_t other_index = __shfl_xor(index, mask, kWave);
-    const bool take = other > value || (other == value && other_index < index);
-    value = take ? other : value;
-    index = take ? other_index : index;
-  }
-  if constexpr (GUARD) exchange_barrier();
-  if (threadIdx.x % kWave == 0) {
-    lds_value[threadIdx.x / kWave] = value;
-    lds_index[threadIdx.x / kWave] = index;
-  }
-  exchange_barrier();
-  T best = lds_value[0];
-  int32_t best_index = lds_index[0];
-#pragma unroll
-  for (int w = 1; w < kWavesPerBlock; ++w) {
-    const T other = lds_value[w];
-    const int32_t other_index = lds_index[w];
-    const bool take = other > best || (other == best && other_index < best_index);
-    best = take ? other : best;
-    best_index = take ? other_index : best_index;
-  }
-  return best;
-}
 
 template <typename T>
 __device__ __forceinline__ T value_max(T a, T b) {
@@ -296,29 +291,52 @@ __device__ __forceinline__ T value_max(T a, T b) {
   }
 }
 
-// Block-wide maximum by value (maxNum: NaN operands are skipped), for a
-// reduction that runs once per kernel (no guard barrier).
-template <typename T, int THREADS>
-__device__ __forceinline__ T block_max_value(T value) {
-  constexpr int kWavesPerBlock = THREADS / kWave;
-  __shared__ T lds_value[kWavesPerBlock];
+// A row's maximum (by value, maxNum: NaN operands are skipped), sum and
+// statistics over its L lanes; every lane gets the result.  A kernel calls
+// each once, so none needs a barrier before its LDS writes.
+template <typename T, int L>
+__device__ __forceinline__ T row_max(T value) {
 #pragma unroll
-  for (int mask = kWave / 2; mask > 0; mask >>= 1) {
+  for (int mask = (L < kWave ? L : kWave) / 2; mask > 0; mask >>= 1) {
     value = value_max(value, __shfl_xor(value, mask, kWave));
   }
-  if (threadIdx.x % kWave == 0) lds_value[threadIdx.x / kWave] = value;
-  exchange_barrier();
-  T best = lds_value[0];
+  if constexpr (L > kWave) {
+    constexpr int kWavesPerBlock = L / kWave;
+    __shared__ T lds_value[kWavesPerBlock];
+    if (threadIdx.x % kWave == 0) lds_value[threadIdx.x / kWave] = value;
+    exchange_barrier();
+    value = lds_value[0];
 #pragma unroll
-  for (int w = 1; w < kWavesPerBlock; ++w) best = value_max(best, lds_value[w]);
-  return best;
+    for (int w = 1; w < kWavesPerBlock; ++w) value = value_max(value, lds_value[w]);
+  }
+  return value;
 }
 
-// Forward over rows held in registers, one row per workgroup (the launcher
-// splits the rows into grids of at most kMaxGrid workgroups).  With no row
-// loop nothing is hoisted across rows, so a lane needs E + ~30 VGPRs and
-// several workgroups share a CU: while one reduces or stores, the others'
-// loads are in flight.
+template <typename T, int L>
+__device__ __forceinline__ T row_sum(T value) {
+  if constexpr (L > kWave) {
+    return block_sum<T, L, false>(value);
+  } else {
+#pragma unroll
+    for (int mask = L / 2; mask > 0; mask >>= 1) value += __shfl_xor(value, mask, kWave);
+    return value;
+  }
+}
+
+template <typename T, int L>
+__device__ __forceinline__ SliceStats<T> row_stats(SliceStats<T> s) {
+  if constexpr (L > kWave) {
+    return block_stats<T, L, false>(s);
+  } else {
+    return lane_stats<T, L>(s);
+  }
+}
+
+// Forward over rows held in registers: L lanes per row, L workgroup-wide or
+// kWave / L rows per single-wave workgroup (the launcher splits the rows into
+// grids of at most kMaxGrid workgroups).  With no row loop nothing is hoisted
+// across rows, so a lane needs E + ~30 VGPRs and several workgroups share a
+// CU: while one reduces or stores, the others' loads are in flight.
 //
 // The fast path keeps no NaN or infinity bookkeeping: with m the maximum
 // over the non-NaN elements, S = sum exp(x - m) is
@@ -328,22 +346,39 @@ __device__ __forceinline__ T block_max_value(T value) {
 // row and apply the reference's special cases from full slice statistics.
 //
 // Waves per SIMD the register budget must allow: a row of up to 128 bytes
-// per lane fits in 64 VGPRs (8 waves, two 1024-lane workgroups per CU);
-// longer rows get 128 (4 waves).
-template <typename T, int E>
+// per lane (and a float32 odd row's one more element) fits in 64 VGPRs (8
+// waves, two 1024-lane workgroups per CU); longer rows get 128 (4 waves).
+template <typename T, int SLOTS>
 constexpr int row_waves() {
-  return sizeof(T) * E <= 128 ? 8 : 4;
+  return sizeof(T) * SLOTS <= 132 ? 8 : 4;
 }
 
-template <typename T, int THREADS, int E, bool LOG, bool VEC, bool FULL, bool NT>
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(row_waves<T, E>())))
-    forward_row_kernel(T* out, int32_t* undefined, const T* in, uint64_t n) {
-  const uint64_t r = blockIdx.x;
-  const int live = FULL ? E : live_slots<T, THREADS, E, VEC>(n);
+template <int L>
+constexpr int row_threads() {
+  return L < kWave ? kWave : L;
+}
+
+template <typename T, int L, int E, bool LOG, int LAYOUT, bool NT>
+__global__ void __launch_bounds__(row_threads<L>())
+    __attribute__((amdgpu_waves_per_eu(row_waves<T, kRowSlots<E, LAYOUT>>())))
+    forward_row_kernel(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n) {
+  constexpr int W = Vec16<T>::width;
+  constexpr int N = kRowSlots<E, LAYOUT>;
+  constexpr uint64_t kRows = row_threads<L>() / L;
+  const uint64_t r = kRows == 1 ? blockIdx.x : blockIdx.x * kRows + threadIdx.x / L;
+  const bool present = kRows == 1 || r < rows;  // the last workgroup's spare lanes hold no row
+  if (!present) n = 0;
+  const int live = LAYOUT == kWhole ? E : live_slots<T, L, E>(n);
   // Slots past the row hold -inf: never a strict maximum, and exp(-inf - m)
   // adds an exact +0 to the sum for every m that leaves the row defined.
-  T x[E];
-  load_row<T, THREADS, E, VEC, FULL>(x, in + r * n, live, -positive_infinity<T>());
+  // Groups of slots past the row in every lane are skipped (E > 32: the row
+  // may leave half of them empty).
+  T x[N];
+  const T* row = in + r * n;
+  load_row<T, L, E, LAYOUT>(x, row, n, live, -positive_infinity<T>());
+  auto used = [&](int j) {
+    return E <= 32 || j >= E || static_cast<uint64_t>(j / W) * L * W < n;
+  };
   // The row maximum over the non-NaN elements, by value only (IEEE maxNum,
   // one v_max per element, which skips NaNs as the CPU's strict `>` scan
   // does).  Which element is the first maximum does not matter here: the
@@ -354,13 +389,13 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(ro
   // that element).
   T lane_max = -positive_infinity<T>();
 #pragma unroll
-  for (int j = 0; j < E; ++j) lane_max = value_max(lane_max, x[j]);
-  // Each block reduction below runs once per kernel: no guard barriers.
-  const T maximum = block_max_value<T, THREADS>(lane_max);
+  for (int j = 0; j < N; ++j) lane_max = value_max(lane_max, x[j]);
+  const T maximum = row_max<T, L>(lane_max);
   // The results overwrite x in place so one row costs E registers per lane.
   T local = T(0);
 #pragma unroll
-  for (int j = 0; j < E; ++j) {
+  for (int j = 0; j < N; ++j) {
+    if (!used(j)) continue;
     if constexpr (LOG) {
       x[j] = x[j] - maximum;
       local += math_exp(x[j]);
@@ -369,141 +404,74 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(ro
       local += x[j];
     }
   }
-  const T total = block_sum<T, THREADS, false>(local);
+  const T total = row_sum<T, L>(local);
   const bool bad = total != total;
-  if (threadIdx.x == 0) undefined[r] = bad ? 1 : 0;
+  if (present && threadIdx.x % L == 0) undefined[r] = bad ? 1 : 0;
   if (!bad) {
     if constexpr (LOG) {
       const T log_sum = math_log(total);
 #pragma unroll
-      for (int j = 0; j < E; ++j) x[j] = x[j] - log_sum;
+      for (int j = 0; j < N; ++j) x[j] = x[j] - log_sum;
     } else {
       const RowDivisor<T> divide(total);
 #pragma unroll
-      for (int j = 0; j < E; ++j) x[j] = divide(x[j]);
+      for (int j = 0; j < N; ++j) {
+        if (used(j)) x[j] = divide(x[j]);
+      }
     }
   } else {
-    load_row<T, THREADS, E, VEC, FULL>(x, in + r * n, live, T(0));
+    load_row<T, L, E, LAYOUT>(x, row, n, live, T(0));
     SliceStats<T> s;
     stats_init(s);
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-      if (FULL || j < live) stats_add(s, x[j], static_cast<int64_t>(column_of<T, THREADS, VEC>(j)));
+    for (int j = 0; j < N; ++j) {
+      const uint32_t column = slot_column<T, L, E>(j, n);
+      const bool held = j < E ? j < live : column < n;
+      if (LAYOUT == kWhole || held) stats_add(s, x[j], static_cast<int64_t>(column));
     }
-    s = block_stats<T, THREADS, false>(s);
+    s = row_stats<T, L>(s);
 #pragma unroll
-    for (int j = 0; j < E; ++j) x[j] = undefined_value<T, LOG>(s, x[j]);
+    for (int j = 0; j < N; ++j) x[j] = undefined_value<T, LOG>(s, x[j]);
   }
-  store_row<T, THREADS, E, VEC, FULL, NT>(out + r * n, x, live);
+  store_row<T, L, E, LAYOUT, NT>(out + r * n, x, n, live);
 }
 
-template <typename T, int THREADS, int E, bool LOG, bool VEC, bool FULL, bool NT>
-__global__ void __launch_bounds__(THREADS)
+template <typename T, int L, int E, bool LOG, int LAYOUT, bool NT>
+__global__ void __launch_bounds__(row_threads<L>())
     backward_row_kernel(T* out, const T* gradient, const T* saved, const int32_t* undefined,
                         uint64_t rows, uint64_t n) {
-  const int live = FULL ? E : live_slots<T, THREADS, E, VEC>(n);
-  for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
-    T* out_row = out + r * n;
-    T g[E];
-    if (undefined[r] != 0) {
+  constexpr int N = kRowSlots<E, LAYOUT>;
+  constexpr uint64_t kRows = row_threads<L>() / L;
+  const uint64_t r = kRows == 1 ? blockIdx.x : blockIdx.x * kRows + threadIdx.x / L;
+  const bool present = kRows == 1 || r < rows;
+  if (!present) n = 0;
+  const int live = LAYOUT == kWhole ? E : live_slots<T, L, E>(n);
+  // Slots past the row hold +0 in both, adding an exact +0 to the sum.
+  T g[N];
+  T y[N];
+  load_row<T, L, E, LAYOUT>(g, gradient + r * n, n, live, T(0));
+  load_row<T, L, E, LAYOUT>(y, saved + r * n, n, live, T(0));
+  const bool bad = present && undefined[r] != 0;
+  T local = T(0);
 #pragma unroll
-      for (int j = 0; j < E; ++j) g[j] = quiet_nan<T>();
-      store_row<T, THREADS, E, VEC, FULL, NT>(out_row, g, live);
-      continue;
-    }
-    // Slots past the row hold +0 in both, adding an exact +0 to the sum.
-    T y[E];
-    load_row<T, THREADS, E, VEC, FULL>(g, gradient + r * n, live, T(0));
-    load_row<T, THREADS, E, VEC, FULL>(y, saved + r * n, live, T(0));
-    T local = T(0);
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      if constexpr (LOG) {
-        local += g[j];
-      } else {
-        local += g[j] * y[j];
-      }
-    }
-    const T reduced = block_sum<T, THREADS>(local);
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      if constexpr (LOG) {
-        g[j] = g[j] - math_exp(y[j]) * reduced;
-      } else {
-        g[j] = y[j] * (g[j] - reduced);
-      }
-    }
-    store_row<T, THREADS, E, VEC, FULL, NT>(out_row, g, live);
-  }
-}
-
-// ------------------------------------------------------ long rows (looped)
-
-constexpr int kLoopThreads = 1024;
-
-template <typename T, bool LOG>
-__global__ void __launch_bounds__(kLoopThreads)
-    forward_loop_kernel(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n) {
-  for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
-    const T* row = in + r * n;
-    T* out_row = out + r * n;
-    SliceStats<T> s;
-    stats_init(s);
-    for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) stats_add(s, row[c], static_cast<int64_t>(c));
-    s = block_stats<T, kLoopThreads>(s);
-    const bool bad = slice_undefined(s);
-    if (threadIdx.x == 0) undefined[r] = bad ? 1 : 0;
-    if (bad) {
-      for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
-        out_row[c] = undefined_value<T, LOG>(s, row[c]);
-      }
-      continue;
-    }
-    const T maximum = s.value;
-    T local = T(0);
-    for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) local += math_exp(row[c] - maximum);
-    const T total = block_sum<T, kLoopThreads>(local);
-    const T log_sum = LOG ? math_log(total) : T(0);
-    const RowDivisor<T> divide(total);
-    for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
-      if constexpr (LOG) {
-        out_row[c] = (row[c] - maximum) - log_sum;
-      } else {
-        out_row[c] = divide(math_exp(row[c] - maximum));
-      }
+  for (int j = 0; j < N; ++j) {
+    if constexpr (LOG) {
+      local += g[j];
+    } else {
+      local += g[j] * y[j];
     }
   }
-}
-
-template <typename T, bool LOG>
-__global__ void __launch_bounds__(kLoopThreads)
-    backward_loop_kernel(T* out, const T* gradient, const T* saved, const int32_t* undefined,
-                         uint64_t rows, uint64_t n) {
-  for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
-    const T* g = gradient + r * n;
-    const T* y = saved + r * n;
-    T* o = out + r * n;
-    if (undefined[r] != 0) {
-      for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) o[c] = quiet_nan<T>();
-      continue;
+  const T reduced = row_sum<T, L>(local);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if constexpr (LOG) {
+      g[j] = g[j] - math_exp(y[j]) * reduced;
+    } else {
+      g[j] = y[j] * (g[j] - reduced);
     }
-    T local = T(0);
-    for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
-      if constexpr (LOG) {
-        local += g[c];
-      } else {
-        local += g[c] * y[c];
-      }
-    }
-    const T reduced = block_sum<T, kLoopThreads>(local);
-    for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
-      if constexpr (LOG) {
-        o[c] = g[c] - math_exp(y[c]) * reduced;
-      } else {
-        o[c] = y[c] * (g[c] - reduced);
-      }
-    }
+    if (bad) g[j] = quiet_nan<T>();
   }
+  store_row<T, L, E, LAYOUT, NT>(out + r * n, g, n, live);
 }
 
 // ------------------------------------------------ running exp-sums
@@ -519,6 +487,199 @@ __device__ __forceinline__ T rescaled(T s, T m, T top) {
 template <typename T>
 __device__ __forceinline__ T exp_term(T x, T top) {
   return x == -positive_infinity<T>() ? T(0) : math_exp(x - top);
+}
+
+// Block-wide merge of the lanes' (m, s): the maximum M of the lane maxima
+// (wave shuffles, then the waves through LDS), then each lane's sum rescaled
+// once by exp(m - M) and the rescaled sums added (wave sums, then in wave
+// order).
+template <typename T, int THREADS>
+__device__ __forceinline__ void block_online(T& m, T& s) {
+  constexpr int kWavesPerBlock = THREADS / kWave;
+  __shared__ T lds_m[kWavesPerBlock];
+  __shared__ T lds_s[kWavesPerBlock];
+  T wave_m = m;
+#pragma unroll
+  for (int mask = kWave / 2; mask > 0; mask >>= 1) {
+    wave_m = value_max(wave_m, __shfl_xor(wave_m, mask, kWave));
+  }
+  const T wave_s = wave_sum(rescaled(s, m, wave_m));
+  exchange_barrier();
+  if (threadIdx.x % kWave == 0) {
+    lds_m[threadIdx.x / kWave] = wave_m;
+    lds_s[threadIdx.x / kWave] = wave_s;
+  }
+  exchange_barrier();
+  T top = lds_m[0];
+#pragma unroll
+  for (int w = 1; w < kWavesPerBlock; ++w) top = value_max(top, lds_m[w]);
+  T total = T(0);
+#pragma unroll
+  for (int w = 0; w < kWavesPerBlock; ++w) total += rescaled(lds_s[w], lds_m[w], top);
+  m = top;
+  s = total;
+}
+
+// ------------------------------------------------------ long rows (looped)
+//
+// Rows past the register budget, 16 bytes per lane at element alignment, four
+// in flight; the n % W last elements go to the first lanes.  The forward keeps
+// a running maximum and rescaled exp-sum per lane and reads the row again for
+// the results: softmax of [256, 70001] float32 takes 38 us, where three scalar
+// reads took 98 us.
+constexpr int kLoopThreads = 1024;
+constexpr int kLoopBatch = 4;
+
+// Walks a lane's part of a row: group(column, B) for B groups, kStep columns
+// apart, and last(column) for its tail element, if it has one.
+template <typename T, typename Group, typename Last>
+__device__ __forceinline__ void walk_row(uint64_t n, Group&& group, Last&& last) {
+  constexpr int W = Vec16<T>::width;
+  constexpr uint64_t kStep = static_cast<uint64_t>(kLoopThreads) * W;
+  const uint64_t body = n / W * W;
+  uint64_t c = static_cast<uint64_t>(threadIdx.x) * W;
+  for (; c + (kLoopBatch - 1) * kStep < body; c += kLoopBatch * kStep) {
+    group(c, std::integral_constant<int, kLoopBatch>{});
+  }
+  for (; c < body; c += kStep) group(c, std::integral_constant<int, 1>{});
+  if (body + threadIdx.x < n) last(body + threadIdx.x);
+}
+
+template <typename T, bool LOG, bool NT>
+__global__ void __launch_bounds__(kLoopThreads)
+    forward_loop_kernel(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n) {
+  constexpr int W = Vec16<T>::width;
+  constexpr uint64_t kStep = static_cast<uint64_t>(kLoopThreads) * W;
+  using V = typename Vec16<T>::type;
+  for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const T* row = in + r * n;
+    T* out_row = out + r * n;
+    T m = -positive_infinity<T>();
+    T s = T(0);
+    auto update = [&](const auto& x) {
+      T top = m;
+      for (const T value : x) top = value_max(top, value);
+      T batch = T(0);
+      for (const T value : x) batch += exp_term(value, top);
+      s = rescaled(s, m, top) + batch;
+      m = top;
+    };
+    walk_row<T>(
+        n,
+        [&](uint64_t c, auto count) {
+          constexpr int B = decltype(count)::value;
+          V v[B];
+#pragma unroll
+          for (int u = 0; u < B; ++u) v[u] = loose_load(row + c + u * kStep);
+          T x[B * W];
+#pragma unroll
+          for (int j = 0; j < B * W; ++j) x[j] = vec_get<T>(v[j / W], j % W);
+          update(x);
+        },
+        [&](uint64_t c) {
+          const T x[1] = {row[c]};
+          update(x);
+        });
+    block_online<T, kLoopThreads>(m, s);
+    const T maximum = m;
+    const T total = s;
+    const bool bad = total != total || maximum == -positive_infinity<T>();
+    if (threadIdx.x == 0) undefined[r] = bad ? 1 : 0;
+    if (bad) {
+      SliceStats<T> stats;
+      stats_init(stats);
+      for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
+        stats_add(stats, row[c], static_cast<int64_t>(c));
+      }
+      stats = block_stats<T, kLoopThreads>(stats);
+      for (uint64_t c = threadIdx.x; c < n; c += kLoopThreads) {
+        out_row[c] = undefined_value<T, LOG>(stats, row[c]);
+      }
+      continue;
+    }
+    const T log_sum = LOG ? math_log(total) : T(0);
+    const RowDivisor<T> divide(total);
+    auto result = [&](T x) {
+      return LOG ? (x - maximum) - log_sum : divide(math_exp(x - maximum));
+    };
+    walk_row<T>(
+        n,
+        [&](uint64_t c, auto count) {
+          constexpr int B = decltype(count)::value;
+          V v[B];
+#pragma unroll
+          for (int u = 0; u < B; ++u) v[u] = loose_load(row + c + u * kStep);
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) vec_set<T>(v[u], k, result(vec_get<T>(v[u], k)));
+            loose_store<NT>(out_row + c + u * kStep, v[u]);
+          }
+        },
+        [&](uint64_t c) { out_row[c] = result(row[c]); });
+  }
+}
+
+template <typename T, bool LOG, bool NT>
+__global__ void __launch_bounds__(kLoopThreads)
+    backward_loop_kernel(T* out, const T* gradient, const T* saved, const int32_t* undefined,
+                         uint64_t rows, uint64_t n) {
+  constexpr int W = Vec16<T>::width;
+  constexpr uint64_t kStep = static_cast<uint64_t>(kLoopThreads) * W;
+  using V = typename Vec16<T>::type;
+  for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const T* g = gradient + r * n;
+    const T* y = saved + r * n;
+    T* o = out + r * n;
+    const bool bad = undefined[r] != 0;
+    T local = T(0);
+    walk_row<T>(
+        n,
+        [&](uint64_t c, auto count) {
+          constexpr int B = decltype(count)::value;
+          V a[B];
+          V b[B];
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            a[u] = loose_load(g + c + u * kStep);
+            if constexpr (!LOG) b[u] = loose_load(y + c + u * kStep);
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+              local += LOG ? vec_get<T>(a[u], k) : vec_get<T>(a[u], k) * vec_get<T>(b[u], k);
+            }
+          }
+        },
+        [&](uint64_t c) { local += LOG ? g[c] : g[c] * y[c]; });
+    const T reduced = block_sum<T, kLoopThreads>(local);
+    auto result = [&](T gv, T yv) {
+      if (bad) return quiet_nan<T>();
+      return LOG ? gv - math_exp(yv) * reduced : yv * (gv - reduced);
+    };
+    walk_row<T>(
+        n,
+        [&](uint64_t c, auto count) {
+          constexpr int B = decltype(count)::value;
+          V a[B];
+          V b[B];
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            a[u] = loose_load(g + c + u * kStep);
+            b[u] = loose_load(y + c + u * kStep);
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+              vec_set<T>(a[u], k, result(vec_get<T>(a[u], k), vec_get<T>(b[u], k)));
+            }
+            loose_store<NT>(o + c + u * kStep, a[u]);
+          }
+        },
+        [&](uint64_t c) { o[c] = result(g[c], y[c]); });
+  }
 }
 
 // -------------------------------------------- non-last axis (inner > 1)
@@ -899,88 +1060,85 @@ uint32_t grid_for(uint64_t blocks) {
   return static_cast<uint32_t>(blocks > kMaxGrid ? kMaxGrid : blocks);
 }
 
-// Register-row configurations (threads, elements per lane), smallest first;
-// FULL drops the bounds checks when the row exactly fills the registers.
-// One workgroup per row, launched in grids of at most kMaxGrid rows.
-template <typename T, int THREADS, int E, bool LOG, bool VEC, bool FULL>
-void forward_rows_as(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n,
-                     const DeviceGuard& guard) {
-  with_policy(stream_output(rows * n * sizeof(T)), [&](auto nt) {
-    constexpr bool NT = decltype(nt)::value;
-    for (uint64_t first = 0; first < rows; first += kMaxGrid) {
-      const uint64_t count = rows - first < kMaxGrid ? rows - first : kMaxGrid;
-      forward_row_kernel<T, THREADS, E, LOG, VEC, FULL, NT>
-          <<<static_cast<uint32_t>(count), THREADS, 0, guard.stream>>>(
-              out + first * n, undefined + first, in + first * n, n);
-    }
-  });
+// A register-row kernel's shape: L lanes per row, E elements per lane.
+template <int L_, int E_>
+struct RowShape {
+  static constexpr int L = L_;
+  static constexpr int E = E_;
+};
+
+// Calls launch(shape, layout, nt, first, rows, grid) for the smallest of the
+// shapes that holds rows of n, in grids of at most kMaxGrid workgroups; false
+// when none does.  Rows that exactly fill a shape of a wave or more drop the
+// bounds checks.
+template <typename T, typename Launch, typename... Shapes>
+bool with_row_shape(uint64_t rows, uint64_t n, bool aligned, Launch&& launch, Shapes... shapes) {
+  constexpr uint64_t W = Vec16<T>::width;
+  auto as = [&](auto shape) {
+    using S = decltype(shape);
+    if (n > static_cast<uint64_t>(S::L) * S::E) return false;
+    constexpr uint64_t kRows = row_threads<S::L>() / S::L;
+    with_policy(stream_output(rows * n * sizeof(T)), [&](auto nt) {
+      auto run = [&](auto layout) {
+        for (uint64_t first = 0; first < rows; first += kMaxGrid * kRows) {
+          const uint64_t count = rows - first < kMaxGrid * kRows ? rows - first : kMaxGrid * kRows;
+          launch(shape, layout, nt, first, count,
+                 static_cast<uint32_t>((count + kRows - 1) / kRows));
+        }
+      };
+      if constexpr (S::L >= kWave && S::E <= 32) {
+        if (aligned && n == static_cast<uint64_t>(S::L) * S::E) {
+          run(std::integral_constant<int, kWhole>{});
+          return;
+        }
+      }
+      if (aligned && n % W == 0) {
+        run(std::integral_constant<int, kGroups>{});
+      } else {
+        run(std::integral_constant<int, kOdd>{});
+      }
+    });
+    return true;
+  };
+  return (as(shapes) || ...);
 }
 
-template <typename T, int THREADS, int E, bool LOG, bool VEC>
-void forward_rows(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n,
-                  const DeviceGuard& guard) {
-  if (n == static_cast<uint64_t>(THREADS) * E) {
-    forward_rows_as<T, THREADS, E, LOG, VEC, true>(out, undefined, in, rows, n, guard);
-  } else {
-    forward_rows_as<T, THREADS, E, LOG, VEC, false>(out, undefined, in, rows, n, guard);
-  }
-}
-
-template <typename T, int THREADS, int E, bool LOG, bool VEC>
-void backward_rows(T* out, const T* gradient, const T* saved, const int32_t* undefined,
-                   uint64_t rows, uint64_t n, const DeviceGuard& guard) {
-  with_policy(stream_output(rows * n * sizeof(T)), [&](auto nt) {
-    constexpr bool NT = decltype(nt)::value;
-    if (n == static_cast<uint64_t>(THREADS) * E) {
-      backward_row_kernel<T, THREADS, E, LOG, VEC, true, NT>
-          <<<grid_for(rows), THREADS, 0, guard.stream>>>(out, gradient, saved, undefined, rows, n);
-    } else {
-      backward_row_kernel<T, THREADS, E, LOG, VEC, false, NT>
-          <<<grid_for(rows), THREADS, 0, guard.stream>>>(out, gradient, saved, undefined, rows, n);
-    }
-  });
-}
-
-// Row lengths up to 1024 take one wave per row (no cross-wave exchange);
-// 8192 takes 256 lanes x 32, which measured faster than 512 x 16.
-template <typename T, bool LOG, bool VEC>
+// Row lengths up to 1024 take one wave or part of one per row (no cross-wave
+// exchange; rows of 8 to 128 were one to a wave and took 14.4 us for 49152 of
+// them, 4.6-8.3 us several to a wave); 8192 takes 256 lanes x 32, which
+// measured faster than 512 x 16.  Up to 65536 float32 stay in registers: 512
+// rows of 50257 take 76 us, where three scalar reads of each took 140 us.
+template <typename T, bool LOG>
 bool launch_forward_rows(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n,
                          const DeviceGuard& guard) {
-  if (n <= 64 * 4) {
-    forward_rows<T, 64, 4, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else if (n <= 64 * 16) {
-    forward_rows<T, 64, 16, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else if (n <= 256 * 16) {
-    forward_rows<T, 256, 16, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else if (n <= 256 * 32) {
-    forward_rows<T, 256, 32, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else if (n <= 1024 * 16) {
-    forward_rows<T, 1024, 16, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else if (n <= 1024 * 32) {
-    forward_rows<T, 1024, 32, LOG, VEC>(out, undefined, in, rows, n, guard);
-  } else {
-    return false;
-  }
-  return true;
+  return with_row_shape<T>(
+      rows, n, aligned16(out) && aligned16(in),
+      [&](auto shape, auto layout, auto nt, uint64_t first, uint64_t count, uint32_t grid) {
+        using S = decltype(shape);
+        forward_row_kernel<T, S::L, S::E, LOG, decltype(layout)::value, decltype(nt)::value>
+            <<<grid, row_threads<S::L>(), 0, guard.stream>>>(out + first * n, undefined + first,
+                                                             in + first * n, count, n);
+      },
+      RowShape<4, 4>{}, RowShape<8, 4>{}, RowShape<16, 4>{}, RowShape<32, 4>{}, RowShape<64, 4>{},
+      RowShape<64, 16>{}, RowShape<256, 16>{}, RowShape<256, 32>{}, RowShape<1024, 16>{},
+      RowShape<1024, 32>{}, RowShape<1024, sizeof(T) == 4 ? 64 : 32>{});
 }
 
-template <typename T, bool LOG, bool VEC>
+template <typename T, bool LOG>
 bool launch_backward_rows(T* out, const T* gradient, const T* saved, const int32_t* undefined,
                           uint64_t rows, uint64_t n, const DeviceGuard& guard) {
-  if (n <= 256 * 4) {
-    backward_rows<T, 256, 4, LOG, VEC>(out, gradient, saved, undefined, rows, n, guard);
-  } else if (n <= 256 * 16) {
-    backward_rows<T, 256, 16, LOG, VEC>(out, gradient, saved, undefined, rows, n, guard);
-  } else if (n <= 512 * 16) {
-    backward_rows<T, 512, 16, LOG, VEC>(out, gradient, saved, undefined, rows, n, guard);
-  } else if (n <= 1024 * 16) {
-    backward_rows<T, 1024, 16, LOG, VEC>(out, gradient, saved, undefined, rows, n, guard);
-  } else if (n <= 1024 * 32) {
-    backward_rows<T, 1024, 32, LOG, VEC>(out, gradient, saved, undefined, rows, n, guard);
-  } else {
-    return false;
-  }
-  return true;
+  return with_row_shape<T>(
+      rows, n, aligned16(out) && aligned16(gradient) && aligned16(saved),
+      [&](auto shape, auto layout, auto nt, uint64_t first, uint64_t count, uint32_t grid) {
+        using S = decltype(shape);
+        backward_row_kernel<T, S::L, S::E, LOG, decltype(layout)::value, decltype(nt)::value>
+            <<<grid, row_threads<S::L>(), 0, guard.stream>>>(out + first * n, gradient + first * n,
+                                                             saved + first * n, undefined + first,
+                                                             count, n);
+      },
+      RowShape<4, 4>{}, RowShape<8, 4>{}, RowShape<16, 4>{}, RowShape<32, 4>{}, RowShape<64, 4>{},
+      RowShape<256, 4>{}, RowShape<256, 16>{}, RowShape<512, 16>{}, RowShape<1024, 16>{},
+      RowShape<1024, 32>{});
 }
 
 // A slice kernel's shape: G slices per unit, X units and Y row groups per
@@ -1009,7 +1167,8 @@ template <typename T, int ARRAYS, typename Launch>
 void launch_slices(uint64_t outer, uint64_t axis, uint64_t inner, const DeviceGuard& guard,
                    Launch&& launch) {
   constexpr int W = Vec16<T>::width;
-  with_policy(stream_output(outer * axis * inner * sizeof(T)), [&](auto nt) {
+  const bool stream = inner % W == 0 && stream_output(outer * axis * inner * sizeof(T));
+  with_policy(stream, [&](auto nt) {
     auto as = [&](auto shape) {
       using S = decltype(shape);
       if constexpr (ARRAYS * S::E * S::G * sizeof(T) <= 256) {
@@ -1051,12 +1210,11 @@ void forward(void* output, int32_t* undefined, const void* input, uint64_t outer
   T* out = static_cast<T*>(output);
   const T* in = static_cast<const T*>(input);
   if (inner == 1) {
-    const bool vec = axis % Vec16<T>::width == 0 && aligned16(out) && aligned16(in);
-    const bool done = vec ? launch_forward_rows<T, LOG, true>(out, undefined, in, outer, axis, guard)
-                          : launch_forward_rows<T, LOG, false>(out, undefined, in, outer, axis, guard);
-    if (!done) {
-      forward_loop_kernel<T, LOG><<<grid_for(outer), kLoopThreads, 0, guard.stream>>>(
-          out, undefined, in, outer, axis);
+    if (!launch_forward_rows<T, LOG>(out, undefined, in, outer, axis, guard)) {
+      with_policy(stream_output(outer * axis * sizeof(T)), [&](auto nt) {
+        forward_loop_kernel<T, LOG, decltype(nt)::value>
+            <<<grid_for(outer), kLoopThreads, 0, guard.stream>>>(out, undefined, in, outer, axis);
+      });
     }
     return;
   }
@@ -1083,13 +1241,12 @@ void backward(void* output, const void* gradient, const void* saved, const int32
   const T* g = static_cast<const T*>(gradient);
   const T* y = static_cast<const T*>(saved);
   if (inner == 1) {
-    const bool vec = axis % Vec16<T>::width == 0 && aligned16(out) && aligned16(g) && aligned16(y);
-    const bool done =
-        vec ? launch_backward_rows<T, LOG, true>(out, g, y, undefined, outer, axis, guard)
-            : launch_backward_rows<T, LOG, false>(out, g, y, undefined, outer, axis, guard);
-    if (!done) {
-      backward_loop_kernel<T, LOG><<<grid_for(outer), kLoopThreads, 0, guard.stream>>>(
-          out, g, y, undefined, outer, axis);
+    if (!launch_backward_rows<T, LOG>(out, g, y, undefined, outer, axis, guard)) {
+      with_policy(stream_output(outer * axis * sizeof(T)), [&](auto nt) {
+        backward_loop_kernel<T, LOG, decltype(nt)::value>
+            <<<grid_for(outer), kLoopThreads, 0, guard.stream>>>(out, g, y, undefined, outer,
+                                                                 axis);
+      });
     }
     return;
   }
@@ -1143,43 +1300,71 @@ constexpr int kEntropyThreads = 256;
 // makes s NaN (NaN - m) and a +inf maximum does too (inf - inf); a row of
 // nothing above -inf keeps m = -inf.  Only the sign of a zero maximum can
 // differ from the first-occurrence rule, which changes no loss or gradient.
-template <typename T> __device__ __forceinline__ T fmax_of(T a, T b);
-template <> __device__ __forceinline__ float fmax_of<float>(float a, float b) { return fmaxf(a, b); }
-template <> __device__ __forceinline__ double fmax_of<double>(double a, double b) { return fmax(a, b); }
+// A row's target, where its loss goes and the logit there.
+template <typename T>
+struct RowTarget {
+  bool present;  // the row has a target
+  bool valid;    // and it is a class
+  uint64_t output_index;
+  T logit;
+};
 
-// Block-wide merge of the lanes' (m, s): the maximum M of the lane maxima
-// (wave shuffles, then the waves through LDS), then each lane's sum rescaled
-// once by exp(m - M) and the rescaled sums added (wave sums, then in wave
-// order).
-template <typename T, int THREADS>
-__device__ __forceinline__ void block_online(T& m, T& s) {
-  constexpr int kWavesPerBlock = THREADS / kWave;
-  __shared__ T lds_m[kWavesPerBlock];
-  __shared__ T lds_s[kWavesPerBlock];
-  T wave_m = m;
-#pragma unroll
-  for (int mask = kWave / 2; mask > 0; mask >>= 1) {
-    wave_m = fmax_of(wave_m, __shfl_xor(wave_m, mask, kWave));
+template <typename T, typename I>
+__device__ __forceinline__ RowTarget<T> row_target(const T* row, const I* targets, uint64_t r,
+                                                   uint64_t classes, TargetMap map) {
+  RowTarget<T> found{};
+  uint64_t target_index;
+  found.present = map.lookup(r, target_index, found.output_index);
+  if (found.present) {
+    const I target = targets[target_index];
+    found.valid = target >= 0 && static_cast<uint64_t>(target) < classes;
+    if (found.valid) found.logit = row[static_cast<uint64_t>(target)];
   }
-  const T wave_s = wave_sum(rescaled(s, m, wave_m));
-  exchange_barrier();
-  if (threadIdx.x % kWave == 0) {
-    lds_m[threadIdx.x / kWave] = wave_m;
-    lds_s[threadIdx.x / kWave] = wave_s;
-  }
-  exchange_barrier();
-  T top = lds_m[0];
-#pragma unroll
-  for (int w = 1; w < kWavesPerBlock; ++w) top = fmax_of(top, lds_m[w]);
-  T total = T(0);
-#pragma unroll
-  for (int w = 0; w < kWavesPerBlock; ++w) total += rescaled(lds_s[w], lds_m[w], top);
-  m = top;
-  s = total;
+  return found;
 }
 
-// Forward: one streaming pass per logits row (non-temporal 16-byte loads,
-// batches of eight per lane) gives the row maximum m and S = sum exp(x - m);
+// What the forward leaves of a row: its statistics for the backward, and the
+// loss, the log-softmax value at the target negated.
+template <typename T>
+struct LossOutputs {
+  T* losses;
+  T* row_max;
+  T* row_log_sum;
+  int32_t* undefined;
+  int32_t* invalid;
+
+  __device__ __forceinline__ void write(uint64_t r, T maximum, T sum, bool bad,
+                                        const SliceStats<T>& stats,
+                                        const RowTarget<T>& target) const {
+    const T log_sum = math_log(sum);
+    undefined[r] = bad ? 1 : 0;
+    row_max[r] = maximum;
+    row_log_sum[r] = log_sum;
+    if (!target.present) return;
+    if (!target.valid) {
+      *invalid = 1;
+      losses[target.output_index] = quiet_nan<T>();
+    } else {
+      const T lp = bad ? undefined_value<T, true>(stats, target.logit)
+                       : (target.logit - maximum) - log_sum;
+      losses[target.output_index] = -lp;
+    }
+  }
+};
+
+// 16 bytes of a logits row: non-temporal from aligned rows, cached from rows
+// of odd length (ODD).
+template <typename T, bool ODD>
+__device__ __forceinline__ typename Vec16<T>::type class_group(const T* at) {
+  if constexpr (ODD) {
+    return loose_load(at);
+  } else {
+    return stream_load(reinterpret_cast<const typename Vec16<T>::type*>(at));
+  }
+}
+
+// Forward: one streaming pass per logits row (non-temporal 16-byte loads at
+// element alignment, batches of eight per lane) gives the row maximum m and S = sum exp(x - m);
 // then loss = -((x_t - m) - log S), the log-softmax value at the target
 // negated, with log-softmax's operations.  S carries the rescaling roundings
 // of the online sum (a few ulp; log-softmax's tolerance covers it).  The
@@ -1188,31 +1373,19 @@ __device__ __forceinline__ void block_online(T& m, T& s) {
 // row has no element above -inf (log-softmax's special cases then apply,
 // from a second read of that row).  An out-of-range target is never read: it
 // sets *invalid.
-template <typename T, typename I, bool VEC>
+template <typename T, typename I, bool ODD>
 __global__ void __launch_bounds__(kEntropyThreads)
-    entropy_forward_kernel(T* losses, T* row_max, T* row_log_sum, int32_t* undefined,
-                           int32_t* invalid, const T* logits, const I* targets, uint64_t rows,
-                           uint64_t classes, TargetMap map) {
-  constexpr int W = VEC ? Vec16<T>::width : 1;
+    entropy_forward_kernel(LossOutputs<T> results, const T* logits, const I* targets,
+                           uint64_t rows, uint64_t classes, TargetMap map) {
+  constexpr int W = Vec16<T>::width;
   constexpr int U = 8;
   using V = typename Vec16<T>::type;
   constexpr uint64_t kStep = static_cast<uint64_t>(kEntropyThreads) * W;
   for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     const T* row = logits + r * classes;
     // lane 0 looks up the target and its logit while the row streams in
-    bool has_target = false;
-    bool target_ok = false;
-    uint64_t output_index = 0;
-    T target_logit = T(0);
-    if (threadIdx.x == 0) {
-      uint64_t target_index;
-      has_target = map.lookup(r, target_index, output_index);
-      if (has_target) {
-        const I target = targets[target_index];
-        target_ok = target >= 0 && static_cast<uint64_t>(target) < classes;
-        if (target_ok) target_logit = row[static_cast<uint64_t>(target)];
-      }
-    }
+    RowTarget<T> target{};
+    if (threadIdx.x == 0) target = row_target(row, targets, r, classes, map);
     T m = -positive_infinity<T>();
     T s = T(0);
     // Batch `start` (the same for every lane) covers columns [start, start +
@@ -1226,30 +1399,25 @@ __global__ void __launch_bounds__(kEntropyThreads)
     auto load_whole = [&](T (&x)[U * W], uint64_t start) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const uint64_t c = start + lane_column + u * kStep;
-        if constexpr (VEC) {
-          const V v = stream_load(reinterpret_cast<const V*>(row + c));
+        const V v = class_group<T, ODD>(row + start + lane_column + u * kStep);
 #pragma unroll
-          for (int k = 0; k < W; ++k) x[u * W + k] = vec_get<T>(v, k);
-        } else {
-          x[u] = row[c];
-        }
+        for (int k = 0; k < W; ++k) x[u * W + k] = vec_get<T>(v, k);
       }
     };
-    auto update = [&](const T (&x)[U * W]) {
+    auto update = [&]<int N>(const T (&x)[N]) {
       T top = m;
 #pragma unroll
-      for (int j = 0; j < U * W; ++j) top = fmax_of(top, x[j]);
+      for (int j = 0; j < N; ++j) top = value_max(top, x[j]);
       // exp(x - top) already gives an exact 0 for x = -inf whenever top is
       // above -inf; only a lane whose elements so far are all -inf (or NaN)
       // needs exp_term's guard against -inf - -inf, so it alone recomputes.
       T batch = T(0);
 #pragma unroll
-      for (int j = 0; j < U * W; ++j) batch += math_exp(x[j] - top);
+      for (int j = 0; j < N; ++j) batch += math_exp(x[j] - top);
       if (top == -positive_infinity<T>()) {
         batch = T(0);
 #pragma unroll
-        for (int j = 0; j < U * W; ++j) batch += exp_term(x[j], top);
+        for (int j = 0; j < N; ++j) batch += exp_term(x[j], top);
       }
       s = rescaled(s, m, top) + batch;
       m = top;
@@ -1284,26 +1452,31 @@ __global__ void __launch_bounds__(kEntropyThreads)
         start += kBatch;
       }
     }
-    // A partial last batch pads with -inf.
-    if (start < classes) {
-      T x[U * W];
+    // The groups of a partial last batch, kPart at a time, padded with -inf.
+    constexpr int kPart = 2;
+    const uint64_t body = classes / W * W;
+    for (; start < body; start += kPart * kStep) {
+      T x[kPart * W];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < kPart; ++u) {
         const uint64_t c = start + lane_column + u * kStep;
-        if (c < classes) {
-          if constexpr (VEC) {
-            const V v = stream_load(reinterpret_cast<const V*>(row + c));
+        if (c < body) {
+          const V v = class_group<T, ODD>(row + c);
 #pragma unroll
-            for (int k = 0; k < W; ++k) x[u * W + k] = vec_get<T>(v, k);
-          } else {
-            x[u] = row[c];
-          }
+          for (int k = 0; k < W; ++k) x[u * W + k] = vec_get<T>(v, k);
         } else {
 #pragma unroll
           for (int k = 0; k < W; ++k) x[u * W + k] = -positive_infinity<T>();
         }
       }
       update(x);
+    }
+    // The classes % W last elements, one per lane.
+    if (body + threadIdx.x < classes) {
+      const T x = row[body + threadIdx.x];
+      const T top = value_max(m, x);
+      s = rescaled(s, m, top) + exp_term(x, top);
+      m = top;
     }
     block_online<T, kEntropyThreads>(m, s);
     const T maximum = m;
@@ -1317,22 +1490,54 @@ __global__ void __launch_bounds__(kEntropyThreads)
       stats = block_stats<T, kEntropyThreads>(stats);
     }
     if (threadIdx.x == 0) {
-      const T log_sum = math_log(s);
-      undefined[r] = bad ? 1 : 0;
-      row_max[r] = maximum;
-      row_log_sum[r] = log_sum;
-      if (has_target) {
-        if (!target_ok) {
-          *invalid = 1;
-          losses[output_index] = quiet_nan<T>();
-        } else {
-          const T lp = bad ? undefined_value<T, true>(stats, target_logit)
-                           : (target_logit - maximum) - log_sum;
-          losses[output_index] = -lp;
-        }
-      }
+      results.write(r, maximum, s, bad, stats, target);
     }
   }
+}
+
+// Rows of up to 4096 classes: held in registers like the softmax forward's (L
+// lanes each, several to a wave where they are short), so the maximum and the
+// exp-sum take one pass each over registers.  In the streaming kernel a row
+// of 10 to 1000 classes was one partly filled batch of a whole workgroup: the
+// loss of [16384, 10] float32 logits took 76 us there and 38 us here, of
+// [4096, 1000] 55 and 37 us, most of what is left its target check's wait.
+template <typename T, typename I, int L, int E, int LAYOUT>
+__global__ void __launch_bounds__(row_threads<L>())
+    entropy_row_kernel(LossOutputs<T> results, const T* logits, const I* targets, uint64_t first,
+                       uint64_t rows, uint64_t classes, TargetMap map) {
+  constexpr int N = kRowSlots<E, LAYOUT>;
+  constexpr uint64_t kRows = row_threads<L>() / L;
+  const uint64_t local_row = kRows == 1 ? blockIdx.x : blockIdx.x * kRows + threadIdx.x / L;
+  const bool present = kRows == 1 || local_row < rows;
+  const uint64_t r = first + local_row;
+  const uint64_t n = present ? classes : 0;
+  const T* row = logits + r * classes;
+  const int live = LAYOUT == kWhole ? E : live_slots<T, L, E>(n);
+  T x[N];
+  load_row<T, L, E, LAYOUT>(x, row, n, live, -positive_infinity<T>());
+  RowTarget<T> target{};
+  if (present && threadIdx.x % L == 0) target = row_target(row, targets, r, classes, map);
+  T maximum = -positive_infinity<T>();
+#pragma unroll
+  for (int j = 0; j < N; ++j) maximum = value_max(maximum, x[j]);
+  maximum = row_max<T, L>(maximum);
+  T sum = T(0);
+#pragma unroll
+  for (int j = 0; j < N; ++j) sum += math_exp(x[j] - maximum);
+  sum = row_sum<T, L>(sum);
+  const bool bad = sum != sum;  // as in the softmax forward
+  SliceStats<T> stats;
+  if (bad) {
+    stats_init(stats);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const uint32_t column = slot_column<T, L, E>(j, n);
+      const bool held = j < E ? j < live : column < n;
+      if (LAYOUT == kWhole || held) stats_add(stats, x[j], static_cast<int64_t>(column));
+    }
+    stats = row_stats<T, L>(stats);
+  }
+  if (present && threadIdx.x % L == 0) results.write(r, maximum, sum, bad, stats, target);
 }
 
 // Backward through NLL and log-softmax at once.  The reference's gradient of
@@ -1346,18 +1551,20 @@ __global__ void __launch_bounds__(kEntropyThreads)
 // fastest; see elementwise.hip).  A lane issues its kEntropyVectors logit
 // loads before the row's statistics loads, so two 16-byte loads per lane are
 // in flight while the row's scalars arrive: 15% faster than one load per
-// lane on [8192, 32768] (bitwise equal).  Tile counts below 2^31 use
+// lane on [8192, 32768] (bitwise equal).  Rows of odd length move 16 bytes at
+// element alignment (their last classes one by one): with scalar accesses,
+// [2048, 50257] float32 took 248 us.  Tile counts below 2^31 use
 // multiply-shift division.
 constexpr int kEntropyTileThreads = 64;
 constexpr int kEntropyVectors = 2;
 
-template <typename T, typename I, bool VEC, bool NT>
+template <typename T, typename I, bool ODD, bool NT>
 __global__ void __launch_bounds__(kEntropyTileThreads)
     entropy_backward_kernel(T* dx, const T* loss_gradient, const T* logits, const T* row_max,
                             const T* row_log_sum, const int32_t* undefined, const I* targets,
                             uint64_t rows, uint64_t classes, uint64_t column_tiles,
                             FastDiv tiles_per_row, TargetMap map) {
-  constexpr int W = VEC ? Vec16<T>::width : 1;
+  constexpr int W = Vec16<T>::width;
   constexpr int U = kEntropyVectors;
   constexpr uint64_t kSpan = static_cast<uint64_t>(kEntropyTileThreads) * W;  // columns per load step
   using V = typename Vec16<T>::type;
@@ -1372,14 +1579,13 @@ __global__ void __launch_bounds__(kEntropyTileThreads)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t c = c0 + u * kSpan;
-      if (c < classes) {
-        if constexpr (VEC) {
-          const V v = stream_load(reinterpret_cast<const V*>(row + c));
+      if (c + W <= classes) {
+        const V v = class_group<T, ODD>(row + c);
 #pragma unroll
-          for (int k = 0; k < W; ++k) values[u][k] = vec_get<T>(v, k);
-        } else {
-          values[u][0] = row[c];
-        }
+        for (int k = 0; k < W; ++k) values[u][k] = vec_get<T>(v, k);
+      } else {
+#pragma unroll
+        for (int k = 0; k < W; ++k) values[u][k] = c + k < classes ? row[c + k] : T(0);
       }
     }
     uint64_t target_index, output_index;
@@ -1402,13 +1608,17 @@ __global__ void __launch_bounds__(kEntropyTileThreads)
         const T g = (c + k == t) ? g_t : T(0);
         values[u][k] = bad ? quiet_nan<T>() : g - math_exp(lp) * g_t;
       }
-      if constexpr (VEC) {
+      T* at = dx + r * classes + c;
+      if (c + W <= classes) {
         V o;
 #pragma unroll
         for (int k = 0; k < W; ++k) vec_set<T>(o, k, values[u][k]);
-        store_vector<NT>(reinterpret_cast<V*>(dx + r * classes + c), o);
+        loose_store<NT>(at, o);
       } else {
-        dx[r * classes + c] = values[u][0];
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+          if (c + k < classes) at[k] = values[u][k];
+        }
       }
     }
   }
@@ -1559,18 +1769,26 @@ void launch_entropy_forward(void* losses, void* row_max, void* row_log_sum,
                             int32_t* undefined_rows, int32_t* invalid, const void* logits,
                             const void* targets, uint64_t rows, uint64_t classes,
                             TargetMap map, const DeviceGuard& guard) {
-  const bool vec = classes % Vec16<T>::width == 0 && aligned16(logits);
-  auto launch = [&](auto kernel) {
-    kernel<<<grid_for(rows), kEntropyThreads, 0, guard.stream>>>(
-        static_cast<T*>(losses), static_cast<T*>(row_max), static_cast<T*>(row_log_sum),
-        undefined_rows, invalid, static_cast<const T*>(logits), static_cast<const I*>(targets),
-        rows, classes, map);
-  };
-  if (vec) {
-    launch(entropy_forward_kernel<T, I, true>);
-  } else {
-    launch(entropy_forward_kernel<T, I, false>);
-  }
+  const LossOutputs<T> results{static_cast<T*>(losses), static_cast<T*>(row_max),
+                               static_cast<T*>(row_log_sum), undefined_rows, invalid};
+  const T* x = static_cast<const T*>(logits);
+  const I* labels = static_cast<const I*>(targets);
+  const bool in_registers = with_row_shape<T>(
+      rows, classes, aligned16(logits),
+      [&](auto shape, auto layout, auto, uint64_t first, uint64_t count, uint32_t grid) {
+        using S = decltype(shape);
+        entropy_row_kernel<T, I, S::L, S::E, decltype(layout)::value>
+            <<<grid, row_threads<S::L>(), 0, guard.stream>>>(results, x, labels, first, count,
+                                                             classes, map);
+      },
+      RowShape<4, 4>{}, RowShape<8, 4>{}, RowShape<16, 4>{}, RowShape<32, 4>{}, RowShape<64, 4>{},
+      RowShape<64, 16>{}, RowShape<256, 16>{});
+  if (in_registers) return;
+  with_policy(classes % Vec16<T>::width != 0 || !aligned16(logits), [&](auto odd) {
+    entropy_forward_kernel<T, I, decltype(odd)::value>
+        <<<grid_for(rows), kEntropyThreads, 0, guard.stream>>>(results, x, labels, rows, classes,
+                                                               map);
+  });
 }
 
 template <typename T, typename I>
@@ -1578,26 +1796,26 @@ void launch_entropy_backward(void* logits_gradient, const void* loss_gradient,
                              const void* logits, const void* row_max, const void* row_log_sum,
                              const int32_t* undefined_rows, const void* targets, uint64_t rows,
                              uint64_t classes, TargetMap map, const DeviceGuard& guard) {
-  const bool vec = classes % Vec16<T>::width == 0 && aligned16(logits) &&
-                   aligned16(logits_gradient);
-  const uint64_t tile_columns = kEntropyTileThreads * (vec ? Vec16<T>::width : 1) * kEntropyVectors;
+  const uint64_t tile_columns = kEntropyTileThreads * Vec16<T>::width * kEntropyVectors;
   const uint64_t column_tiles = (classes + tile_columns - 1) / tile_columns;
   FastDiv tiles_per_row;
   tiles_per_row.init(column_tiles <= kIndex32Limit ? static_cast<uint32_t>(column_tiles) : 1U);
-  auto launch = [&](auto kernel) {
-    kernel<<<grid_for(rows * column_tiles), kEntropyTileThreads, 0, guard.stream>>>(
-        static_cast<T*>(logits_gradient), static_cast<const T*>(loss_gradient),
-        static_cast<const T*>(logits), static_cast<const T*>(row_max),
-        static_cast<const T*>(row_log_sum), undefined_rows, static_cast<const I*>(targets), rows,
-        classes, column_tiles, tiles_per_row, map);
+  auto launch = [&](auto odd, auto nt) {
+    entropy_backward_kernel<T, I, decltype(odd)::value, decltype(nt)::value>
+        <<<grid_for(rows * column_tiles), kEntropyTileThreads, 0, guard.stream>>>(
+            static_cast<T*>(logits_gradient), static_cast<const T*>(loss_gradient),
+            static_cast<const T*>(logits), static_cast<const T*>(row_max),
+            static_cast<const T*>(row_log_sum), undefined_rows, static_cast<const I*>(targets),
+            rows, classes, column_tiles, tiles_per_row, map);
   };
-  if (vec) {
-    with_policy(stream_output(rows * classes * sizeof(T)), [&](auto nt) {
-      launch(entropy_backward_kernel<T, I, true, decltype(nt)::value>);
-    });
-  } else {
-    launch(entropy_backward_kernel<T, I, false, false>);
-  }
+  // (Odd rows keep non-temporal stores: with ordinary ones the backward over
+  // [2048, 50257] float32 took 140 us instead of 154, but the dirty lines it
+  // left in cache put 37 us on the next forward.)
+  const bool odd_rows =
+      classes % Vec16<T>::width != 0 || !aligned16(logits) || !aligned16(logits_gradient);
+  with_policy(odd_rows, [&](auto odd) {
+    with_policy(stream_output(rows * classes * sizeof(T)), [&](auto nt) { launch(odd, nt); });
+  });
 }
 
 bool entropy_geometry_ok(uint64_t rows, uint64_t classes, uint64_t sequence_length,

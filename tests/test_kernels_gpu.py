@@ -1168,6 +1168,61 @@ def test_softmax_rows_beyond_one_grid(hip):
     assert np.all(np.isnan(got[-1]))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 63, 65, 127, 129, 255, 257, 1023,
+                               1025, 4097, 8191, 16385, 32769, 65535, 65537])
+def test_softmax_odd_rows(hip, dtype, n):
+    """Rows of any length from a misaligned start, several to a wave where
+    they are short, with undefined rows beside defined ones: the register
+    shapes' edges, their one-by-one last elements and the looped rows."""
+    rows = 67 if n < 2000 else 6
+    x = (inputs(65, rows * n, dtype, with_specials=False) * dtype(1.5)).reshape(rows, n)
+    x[1, n // 2] = np.nan
+    x[2, :] = -np.inf
+    x[3, n - 1] = np.inf
+    x[5, 0] = -np.inf if n > 1 else 0.0
+    g = inputs(66, rows * n, dtype, with_specials=False).reshape(rows, n)
+
+    def misaligned(a):
+        item = np.dtype(dtype).itemsize
+        buffer = hip.DeviceBuffer(a.nbytes + 2 * item)
+        hip.call("spar_hip_copy_host_to_device", buffer.address(item),
+                 np.ascontiguousarray(a).ctypes.data, a.nbytes, 0)
+        return buffer, buffer.address(item)
+
+    for log in (False, True):
+        want, und_ref = (ref.log_softmax(x, 1) if log else ref.softmax_axis(x, 1))
+        flags = und_ref.astype(np.int32)
+        source, source_at = misaligned(x)
+        out, out_at = misaligned(np.zeros_like(x))
+        undefined = out_buf(hip, (rows,), np.int32)
+        hip.call("spar_hip_launch_probability_forward", out_at, undefined.ptr, source_at, rows, n, 1,
+                 tag(dtype), int(log), 0)
+        got = np.empty_like(x)
+        hip.call("spar_hip_copy_device_to_host", got.ctypes.data, out_at, got.nbytes, 0)
+        assert np.array_equal(undefined.to_numpy(np.int32, (rows,)), flags)
+        defined = np.broadcast_to((flags == 0)[:, None], x.shape)
+        assert_ulp(got[~defined], want[~defined], 2, f"undefined rows n={n} log={log}")
+        check = log_softmax_tolerance_check if log else softmax_tolerance_check
+        check(got[flags == 0], want[flags == 0], n, dtype, f"odd rows n={n} log={log}")
+        saved, saved_at = misaligned(want)
+        gradient, gradient_at = misaligned(g)
+        hip.call("spar_hip_launch_probability_backward", out_at, gradient_at, saved_at,
+                 undefined.ptr, rows, n, 1, tag(dtype), int(log), 0)
+        back = np.empty_like(x)
+        hip.call("spar_hip_copy_device_to_host", back.ctypes.data, out_at, back.nbytes, 0)
+        assert np.array_equal(np.isnan(back), ~defined)
+        y = np.where(defined, want, 0).astype(np.float64)
+        gd = g.astype(np.float64)
+        p = np.exp(y) if log else y
+        s = gd.sum(1, keepdims=True) if log else (gd * y).sum(1, keepdims=True)
+        exact = gd - p * s if log else y * (gd - s)
+        magnitude = (np.abs(gd) if log else np.abs(gd * y)).sum(1, keepdims=True)
+        u = np.finfo(dtype).eps  # an n-long sum, then a few roundings
+        bound = (n + 8) * u * p * magnitude + 4 * u * (np.abs(gd) + np.abs(exact))
+        assert (np.abs(back.astype(np.float64) - exact) <= bound)[defined].all(), f"n={n} log={log}"
+
+
 # [outer, axis, inner] at the edges of the slice kernels' shapes: 16-byte units
 # (inner from 32 on, also not a multiple of the vector) and single slices, rows
 # per lane group full, partial and one past, few and many workgroups, looped.
