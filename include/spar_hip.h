@@ -223,6 +223,15 @@ struct SparHipStatus spar_hip_launch_scalar(void* output, const void* input, uin
 struct SparHipStatus spar_hip_launch_unary(void* output, const void* input, uint64_t count,
                                            int dtype, int operation, int device);
 
+/* output[i] = gradient[i] * op'(saved[i]) for SQUARE, RECIPROCAL, SILU and
+ * GELU (saved: the op's input) and SQRT, SIGMOID and TANH (saved: its output):
+ * the backward chains of src/ops/unary.cpp:55-164 in one pass, each operation
+ * rounded as the separate ops round it.  The other ops have no such form
+ * (status 1).  No reference counterpart. */
+struct SparHipStatus spar_hip_launch_unary_backward(void* output, const void* gradient,
+                                                    const void* saved, uint64_t count, int dtype,
+                                                    int operation, int device);
+
 /* output[i] = scalar[0] * (T)scale, with scalar a device pointer to one
  * element: the reference's semantics.  Replaces
  * spar_cuda_launch_fill_from_scalar (cuda_kernels.hpp:85-87,

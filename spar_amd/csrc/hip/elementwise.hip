@@ -29,7 +29,6 @@ namespace {
 // with workgroups of 64 / 128 / 256 / 512 lanes.
 constexpr int kThreads = 256;        // grid-stride scalar kernels
 constexpr int kVectorThreads = 64;   // streaming vector kernels
-constexpr int kUnroll = 1;
 constexpr uint64_t kMaxGrid = uint64_t{1} << 20;
 
 template <typename T, typename F, bool NT>
@@ -72,17 +71,18 @@ __global__ void __launch_bounds__(kVectorThreads)
     map2_vec_kernel(T* out, const T* a, const T* b, uint64_t count, F f) {
   using V = typename Vec16<T>::type;
   constexpr int W = Vec16<T>::width;
+  constexpr int U = VectorsPerLane<F>::value;
   const uint64_t vectors = count / W;
-  const uint64_t tile = static_cast<uint64_t>(kVectorThreads) * kUnroll;
+  const uint64_t tile = static_cast<uint64_t>(kVectorThreads) * U;
   const V* a_v = reinterpret_cast<const V*>(a);
   const V* b_v = reinterpret_cast<const V*>(b);
   V* out_v = reinterpret_cast<V*>(out);
   for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * tile; base < vectors;
        base += static_cast<uint64_t>(gridDim.x) * tile) {
-    V ra[kUnroll];
-    V rb[kUnroll];
+    V ra[U];
+    V rb[U];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const uint64_t i = base + static_cast<uint64_t>(u) * kVectorThreads + threadIdx.x;
       if (i < vectors) {
         ra[u] = stream_load(a_v + i);
@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(kVectorThreads)
       }
     }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const uint64_t i = base + static_cast<uint64_t>(u) * kVectorThreads + threadIdx.x;
       if (i < vectors) {
         V o;
@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-uint32_t vector_grid(uint64_t count, int width, int vectors_per_lane = kUnroll) {
+uint32_t vector_grid(uint64_t count, int width, int vectors_per_lane = 1) {
   const uint64_t vectors = count / static_cast<uint64_t>(width);
   const uint64_t tile = static_cast<uint64_t>(kVectorThreads) * vectors_per_lane;
   uint64_t blocks = (vectors + tile - 1) / tile;
@@ -262,8 +262,8 @@ void launch_map2(T* out, const T* a, const T* b, uint64_t count, F f, const Devi
   if (aligned16(out) && aligned16(a) && aligned16(b)) {
     with_policy(stream_output(count * sizeof(T)), [&](auto nt) {
       map2_vec_kernel<T, F, decltype(nt)::value>
-          <<<vector_grid(count, Vec16<T>::width), kVectorThreads, 0, guard.stream>>>(out, a, b,
-                                                                                    count, f);
+          <<<vector_grid(count, Vec16<T>::width, VectorsPerLane<F>::value), kVectorThreads, 0,
+             guard.stream>>>(out, a, b, count, f);
     });
   } else {
     map2_scalar_kernel<T, F><<<scalar_grid(count, guard), kThreads, 0, guard.stream>>>(
@@ -687,6 +687,28 @@ extern "C" SparHipStatus spar_hip_launch_unary(void* output, const void* input, 
     } else {
       launch_map1(static_cast<double*>(output), static_cast<const double*>(input), count, op,
                   guard);
+    }
+  });
+  return finish(guard);
+}
+
+extern "C" SparHipStatus spar_hip_launch_unary_backward(void* output, const void* gradient,
+                                                        const void* saved, uint64_t count,
+                                                        int dtype, int operation, int device) {
+  if (!valid_float_dtype(dtype) || !dispatch_unary_gradient(operation, [](auto) {}) ||
+      (count != 0 && (output == nullptr || gradient == nullptr || saved == nullptr))) {
+    return invalid();
+  }
+  if (count == 0) return ok();
+  DeviceGuard guard;
+  if (enter(device, guard) != hipSuccess) return runtime(guard.error);
+  dispatch_unary_gradient(operation, [&](auto op) {
+    if (dtype == SPAR_HIP_FLOAT32) {
+      launch_map2(static_cast<float*>(output), static_cast<const float*>(gradient),
+                  static_cast<const float*>(saved), count, op, guard);
+    } else {
+      launch_map2(static_cast<double*>(output), static_cast<const double*>(gradient),
+                  static_cast<const double*>(saved), count, op, guard);
     }
   });
   return finish(guard);

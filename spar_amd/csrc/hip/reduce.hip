@@ -390,8 +390,8 @@ __global__ void __launch_bounds__(kThreads)
 // order with the exact rule, as row_kernel does.  On 2^25 float32 elements
 // the sum over 512 such blocks and the combine took 22.8 us against 25.1 us
 // for 2048 blocks each scanning a contiguous 64 KiB segment, and on 2^28
-// 156-162 us against 172 us on the same box.  The row's start and length
-// are multiples of W.
+// 156-162 us against 172 us on the same box.  The row's start is a multiple of
+// W; the n % W last elements go to the last block's first lanes.
 constexpr uint64_t kInterleavedBlocksPerCu = 2;
 
 template <typename T, Kind K, int NIN>
@@ -444,6 +444,11 @@ __global__ void __launch_bounds__(kThreads)
         for (int k = 0; k < W; ++k) scan[0].add(vec_get<T>(v, k), element + k);
       }
     }
+  }
+  // past every element of the lane, by the exact rule
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x < n % W) {
+    const uint64_t element = vectors * W + threadIdx.x;
+    scan[0].add(load_value<T, NIN>(a, b, base + element), static_cast<uint32_t>(element));
   }
   Acc<T, K> acc[4];
 #pragma unroll
@@ -1346,8 +1351,10 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     }
     const uint64_t range_splits = (n + kMaxScanRange / 2 - 1) / (kMaxScanRange / 2);
     if (splits < range_splits) splits = range_splits;
-    // A full reduction of a long contiguous row: interleaved blocks.
-    if (rows == 1 && vec && splits > 1 && n < kMaxScanRange) {
+    // A full reduction of a long contiguous row: interleaved blocks (of any
+    // length: [2047, 2731] float32 summed by scalar segments took 12.7 us).
+    const bool start_aligned = plan.offset % W == 0 && aligned16(a) && (NIN == 1 || aligned16(b));
+    if (rows == 1 && start_aligned && splits > 1 && n < kMaxScanRange) {
       uint64_t blocks = static_cast<uint64_t>(cus) * kInterleavedBlocksPerCu;
       if (blocks > splits) blocks = splits;
       const uint64_t base = map.offset;  // row 0

@@ -170,6 +170,23 @@ Tensor dispatch_unary(const Tensor& input, int operation, const char* name) {
   return output;
 }
 
+// gradient * op'(saved) in one pass, or nothing when the gradient is a view
+// (a reduction's broadcast), which the chain of ops reads in place.
+std::optional<Tensor> unary_gradient(const Tensor& gradient, const Tensor& saved, int operation,
+                                     const char* name) {
+  if (!gradient.device().is_hip() || !full_contiguous(gradient, saved.shape()) ||
+      !saved.is_contiguous() || gradient.numel() == 0) {
+    return std::nullopt;
+  }
+  Tensor result{saved.shape(), saved.dtype(), saved.device()};
+  hip::check(spar_hip_launch_unary_backward(
+                 HipTensorAccess::mutable_data(result), HipTensorAccess::data(gradient),
+                 HipTensorAccess::data(saved), saved.numel(), hip::dtype_tag(saved.dtype()),
+                 operation, saved.device().index()),
+             name, saved.device());
+  return result;
+}
+
 }  // namespace
 
 // ------------------------------------------------------------ elementwise
@@ -344,6 +361,9 @@ Tensor square(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_input{input.detach()};
     detail::record_operation(output, {input}, [saved_input](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_input, SPAR_HIP_SQUARE, "square backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       return std::vector<Tensor>{multiply(gradient, multiply_scalar(saved_input, 2.0))};
     });
   }
@@ -355,6 +375,9 @@ Tensor reciprocal(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_input{input.detach()};
     detail::record_operation(output, {input}, [saved_input](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_input, SPAR_HIP_RECIPROCAL, "reciprocal backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       const auto denominator{multiply(saved_input, saved_input)};
       return std::vector<Tensor>{multiply_scalar(divide(gradient, denominator), -1.0)};
     });
@@ -389,6 +412,9 @@ Tensor sqrt(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_output{output.detach()};
     detail::record_operation(output, {input}, [saved_output](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_output, SPAR_HIP_SQRT, "sqrt backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       return std::vector<Tensor>{divide(gradient, multiply_scalar(saved_output, 2.0))};
     });
   }
@@ -400,6 +426,9 @@ Tensor sigmoid(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_output{output.detach()};
     detail::record_operation(output, {input}, [saved_output](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_output, SPAR_HIP_SIGMOID, "sigmoid backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       const auto one_minus_output{add_scalar(multiply_scalar(saved_output, -1.0), 1.0)};
       return std::vector<Tensor>{multiply(gradient, multiply(saved_output, one_minus_output))};
     });
@@ -412,6 +441,9 @@ Tensor silu(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_input{input.detach()};
     detail::record_operation(output, {input}, [saved_input](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_input, SPAR_HIP_SILU, "silu backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       // unary.cpp:155-160
       const auto sigmoid_value{sigmoid(saved_input)};
       const auto one_minus_sigmoid{add_scalar(multiply_scalar(sigmoid_value, -1.0), 1.0)};
@@ -429,6 +461,9 @@ Tensor tanh(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_output{output.detach()};
     detail::record_operation(output, {input}, [saved_output](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_output, SPAR_HIP_TANH, "tanh backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       const auto one_minus_square{
           add_scalar(multiply_scalar(multiply(saved_output, saved_output), -1.0), 1.0)};
       return std::vector<Tensor>{multiply(gradient, one_minus_square)};
@@ -443,6 +478,9 @@ Tensor gelu(const Tensor& input) {
   if (input.requires_grad()) {
     const Tensor saved_input{input.detach()};
     detail::record_operation(output, {input}, [saved_input](const Tensor& gradient) {
+      if (auto fused{unary_gradient(gradient, saved_input, SPAR_HIP_GELU, "gelu backward")}) {
+        return std::vector<Tensor>{*std::move(fused)};
+      }
       const auto slope{dispatch_unary(saved_input, SPAR_HIP_GELU_DERIVATIVE, "gelu backward")};
       return std::vector<Tensor>{multiply(gradient, slope)};
     });

@@ -107,6 +107,82 @@ def test_unary(hip, dtype, op):
         assert_ulp(got, want, 4 if (dtype == F64 and composite) else 2, op)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [1, 3, 5, 255, 257, 511, 513, 1029, 200003])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_unary_backward_matches_the_chain(hip, dtype, n, offset):
+    """Each fused gradient gives the bits of its chain of separate ops, edge
+    values, tails and misaligned pointers included."""
+    with np.errstate(over="ignore"):
+        x = inputs(5, n + 1, dtype) * dtype(2)
+    g = inputs(6, n + 1, dtype)
+    size = np.dtype(dtype).itemsize
+    kept = [dev(hip, x), dev(hip, g)]
+    x_at, g_at = (b.address(offset * size) for b in kept)
+
+    def buffer():
+        return out_buf(hip, (n + 1,), dtype).address(offset * size)
+
+    def unary(a, op):
+        out = buffer()
+        hip.call("spar_hip_launch_unary", out, a, n, tag(dtype), hip.UNARY_OPS[op], 0)
+        return out
+
+    def scalar(a, op, value):
+        out = buffer()
+        hip.call("spar_hip_launch_scalar", out, a, n, tag(dtype), hip.BINARY_OPS[op], value, 0)
+        return out
+
+    def binary(a, b, op):
+        out = buffer()
+        hip.call("spar_hip_launch_binary", out, a, b, n, tag(dtype), hip.BINARY_OPS[op], 0)
+        return out
+
+    def one_minus(a):
+        return scalar(scalar(a, "multiply", -1.0), "add", 1.0)
+
+    s = unary(x_at, "sigmoid")
+    slope = binary(s, one_minus(s), "multiply")
+    chains = {
+        "square": binary(g_at, scalar(x_at, "multiply", 2.0), "multiply"),
+        "reciprocal": scalar(binary(g_at, binary(x_at, x_at, "multiply"), "divide"), "multiply",
+                             -1.0),
+        "sqrt": binary(g_at, scalar(x_at, "multiply", 2.0), "divide"),
+        "sigmoid": binary(g_at, binary(x_at, one_minus(x_at), "multiply"), "multiply"),
+        "silu": binary(g_at, binary(s, binary(x_at, slope, "multiply"), "add"), "multiply"),
+        "tanh": binary(g_at, one_minus(binary(x_at, x_at, "multiply")), "multiply"),
+        "gelu": binary(g_at, unary(x_at, "gelu_derivative"), "multiply"),
+    }
+
+    def host(at):
+        out = np.empty(n, dtype)
+        hip.call("spar_hip_copy_device_to_host", out.ctypes.data, at, out.nbytes, 0)
+        return out
+
+    for op, chain in chains.items():
+        fused = buffer()
+        hip.call("spar_hip_launch_unary_backward", fused, g_at, x_at, n, tag(dtype),
+                 hip.UNARY_OPS[op], 0)
+        assert_bitexact(host(fused), host(chain), f"{op} backward n={n} offset={offset}")
+    assert hip.status_of("spar_hip_launch_unary_backward", buffer(), g_at, x_at, n, tag(dtype),
+                         hip.UNARY_OPS["exp"], 0).code == 1
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [65537, 131073, 131075, (1 << 20) + 1, (1 << 20) + 3])
+def test_full_reduction_odd_length(hip, dtype, n):
+    """Long contiguous reductions whose length is no multiple of the vector:
+    the last elements hold the maximum, a tie or the only NaN."""
+    base = inputs(7, n, dtype, with_specials=False)
+    check_axis(hip, base, base, [0], dtype, f"full n={n}")
+    for last in (base.max(), dtype(9.0), dtype(np.nan)):
+        x = base.copy()
+        x[-1] = last
+        mx, am = ref.axis_max(x, [0])
+        assert_bitexact(axis_reduce(hip, x, x, [0], "max", dtype), mx, f"max n={n} {last}")
+        assert_bitexact(axis_reduce(hip, x, x, [0], "argmax", dtype), am, f"argmax n={n} {last}")
+
+
 def test_gelu_float32_sweep(hip):
     """Every 256th float32 bit pattern (2^24 inputs spanning every exponent
     and both signs, with the infinities and NaNs) through GELU and its
