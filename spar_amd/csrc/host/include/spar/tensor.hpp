@@ -293,6 +293,9 @@ void set_scaled_backward(Tensor& output, ScaledBackward scaled);
 /// and the input's producer has a scaled form, the engine hands that
 /// producer (factor, value) instead of running this operation's rule.
 void set_product_factor(Tensor& output, Tensor factor);
+/// Marks `output`'s recorded operation as a plain sum, whose rule broadcasts
+/// the output gradient over its input without reading it.
+void set_broadcasting(Tensor& output);
 void record_transfer_operation(Tensor& output, Tensor requiring_parent, BackwardFunction backward);
 [[nodiscard]] bool shares_autograd_identity(const Tensor& left, const Tensor& right) noexcept;
 

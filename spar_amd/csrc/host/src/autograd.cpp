@@ -32,6 +32,12 @@
 //      rounding and operand order, so x's producer computes what it would
 //      from the materialised product, and every identity still receives its
 //      gradients in the same order.
+//   7. A sweep starts from ones, and a sum hands its input the gradient it
+//      gets, broadcast.  Where the gradient of a product with one tracked
+//      input is therefore known to be all ones, that input's gradient is the
+//      other operand itself (1 * v is v, bit for bit): it is handed on, and no
+//      product is formed.  The ones themselves are written only when a rule
+//      reads them.
 // Given identical contributions, the gradients are therefore identical to
 // the reference's.  The reference also cloned each contribution
 // (autograd.cpp:145, :244), which copied values into a dense tensor.  Here a
@@ -124,6 +130,14 @@ void set_product_factor(Tensor& output, Tensor factor) {
   }
   if (factor.requires_grad()) throw std::logic_error{"A product factor must be detached"};
   state->producer->product_factor = std::move(factor);
+}
+
+void set_broadcasting(Tensor& output) {
+  const auto& state{TensorInternals::grad_state(output)};
+  if (state == nullptr || state->producer == nullptr) {
+    throw std::logic_error{"A broadcasting rule needs a recorded operation"};
+  }
+  state->producer->broadcasts = true;
 }
 
 void record_transfer_operation(Tensor& output, Tensor requiring_parent, BackwardFunction backward) {
@@ -241,8 +255,17 @@ class Sweep final {
     order_from(loss);
   }
 
-  void run(GradState* loss, Tensor seed) {
-    pending_[slot_.at(loss)] = std::move(seed);
+  // Sweeps from a gradient of ones for `loss`, shaped as `shape`.
+  void run(GradState* loss, const Shape& shape, DType dtype, Device device) {
+    const std::size_t first{slot_.at(loss)};
+    if (hand_overs_ && device.is_hip() && loss->producer != nullptr &&
+        loss->producer->broadcasts) {
+      seed_.emplace(shape, dtype, device);  // written when a rule reads it
+      pending_[first] = seed_->detach();
+      ones_[first] = true;
+    } else {
+      pending_[first] = ones(shape, dtype, device);
+    }
     for (std::size_t position{order_.size()}; position-- > 0;) {
       GradState& state{*order_[position]};
       std::optional<Tensor>& held{pending_[position]};
@@ -251,6 +274,17 @@ class Sweep final {
       }
       Tensor gradient{std::move(*held)};
       held.reset();
+      if (ones_[position]) {
+        if (state.producer != nullptr && state.producer->broadcasts &&
+            gradient.is_contiguous()) {
+          propagate(*state.producer, std::move(gradient));
+          const auto below{slot_.find(state.producer->inputs.front().identity.get())};
+          if (below != slot_.end()) ones_[below->second] = incoming_[below->second] == 1;
+          continue;
+        }
+        if (state.producer != nullptr && hand_factor(*state.producer)) continue;
+        write_seed();
+      }
       if (state.producer == nullptr) {
         deliver_to_leaf(state, std::move(gradient));
         continue;
@@ -306,6 +340,7 @@ class Sweep final {
     deferred_.resize(order_.size());
     placed_.resize(order_.size());
     scale_.resize(order_.size());
+    ones_.assign(order_.size(), false);
     incoming_.assign(order_.size(), 0);
     for (const GradState* state : order_) {
       if (state->producer == nullptr) continue;
@@ -410,6 +445,37 @@ class Sweep final {
     scale_[next] = std::move(value);
     g_scaled_gradients.fetch_add(1, std::memory_order_relaxed);
     return true;
+  }
+
+  // Contract, point 7: the product `function`, whose gradient is all ones,
+  // hands its input the other operand.  Not where the input takes more than
+  // this gradient, is a leaf (which would copy it) or has a scaled form (which
+  // takes the product as hand_scaled hands it over), nor where gradients'
+  // zero signs are to be the reference's.
+  bool hand_factor(const GradFunction& function) {
+    if (!function.product_factor.has_value() || exact_gradient_zero_signs()) return false;
+    const GradInput& input{function.inputs.front()};
+    const Tensor& factor{*function.product_factor};
+    const auto found{slot_.find(input.identity.get())};
+    if (found == slot_.end()) return false;
+    const GradFunction* consumer{order_[found->second]->producer.get()};
+    if (consumer == nullptr || consumer->scaled || incoming_[found->second] != 1 ||
+        factor.shape() != input.shape || factor.dtype() != input.dtype ||
+        factor.device() != input.device) {
+      return false;
+    }
+    accumulate(input, factor.detach());
+    return true;
+  }
+
+  // Fills the sweep's seed, once.
+  void write_seed() {
+    if (!seed_.has_value()) return;
+    hip::check(spar_hip_launch_fill(HipTensorAccess::mutable_data(*seed_), seed_->numel(),
+                                    hip::dtype_tag(seed_->dtype()), 1.0,
+                                    seed_->device().index()),
+               "backward", seed_->device());
+    seed_.reset();
   }
 
   struct Placement {
@@ -567,6 +633,10 @@ class Sweep final {
   // per identity: the one value its pending gradient (then a product
   // factor) is to be multiplied by, when a product handed it over scaled
   std::vector<std::optional<Tensor>> scale_;
+  // per identity: its pending gradient is the seed's ones, broadcast
+  std::vector<bool> ones_;
+  // the seed while its ones are still to be written
+  std::optional<Tensor> seed_;
 };
 
 }  // namespace
@@ -622,7 +692,7 @@ void Tensor::backward() {
   }
   detail::g_backward_calls.fetch_add(1, std::memory_order_relaxed);
   detail::Sweep sweep{grad_state_.get()};
-  sweep.run(grad_state_.get(), ones(shape_, dtype_, device()));
+  sweep.run(grad_state_.get(), shape_, dtype_, device());
 }
 
 }  // namespace spar

@@ -51,6 +51,9 @@ struct GradFunction final {
   /// Set for a product with one tracked input: the other operand, which
   /// times the output gradient is that input's gradient.
   std::optional<Tensor> product_factor;
+  /// Set for a plain sum: the rule gives its input the output gradient
+  /// broadcast, reading none of its values.
+  bool broadcasts{false};
 };
 
 struct GradState final {

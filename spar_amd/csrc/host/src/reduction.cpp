@@ -154,6 +154,7 @@ Tensor sum(const Tensor& input) {
     detail::record_operation(output, {input}, [input_shape](const Tensor& gradient) {
       return std::vector<Tensor>{broadcast_full_gradient(input_shape, gradient, std::nullopt)};
     });
+    detail::set_broadcasting(output);
   }
   return output;
 }
@@ -171,6 +172,7 @@ Tensor sum(const Tensor& input, std::span<const std::size_t> axes, bool keepdim)
                                    gradient, input_shape, normalized_axes, keepdim,
                                    std::nullopt)};
                              });
+    detail::set_broadcasting(output);
   }
   return output;
 }

@@ -792,3 +792,48 @@ def test_layernorm_chain_second_run_allocates_nothing_and_copies_no_gradient(sp)
     assert counters_after["in_place_adds"] > counters_before["in_place_adds"]
     for a, b in zip(first, second):
         assert_bitexact(b, a, "second run")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_autograd_ones_handed_through_products(sp, dtype):
+    """A product under plain sums hands its one tracked input the other
+    operand, and the seed's ones are written only where a rule reads them: the
+    gradients' bits are those of the plain rules, the operand itself is left
+    alone, and accumulated or shared gradients are not the operand's storage."""
+    rng = np.random.default_rng(71)
+    device = sp.Device.hip(0)
+    a, c = (rng.standard_normal((33, 65)).astype(dtype) for _ in range(2))
+    c[0, :4] = [0.0, -0.0, np.inf, np.nan]
+
+    def tensor(values, tracked=False):
+        t = sp.Tensor.from_numpy(values).to(device)
+        if tracked:
+            t.set_requires_grad(True)
+        return t
+
+    losses = {
+        "activation": lambda x, g: sp.sum(sp.multiply(sp.silu(x), g)),
+        "operand first": lambda x, g: sp.sum(sp.multiply(g, sp.tanh(x))),
+        "sum of sums": lambda x, g: sp.sum(sp.sum(sp.multiply(sp.exp(x), g), 1)),
+        "leaf": lambda x, g: sp.sum(sp.multiply(x, g)),
+        "passed on": lambda x, g: sp.sum(sp.multiply(sp.add(x, x), g)),
+        "shared": lambda x, g: sp.sum(sp.multiply(sp.add_scalar(sp.add(x, sp.square(x)), 1.0), g)),
+        "two products": lambda x, g: sp.add(sp.sum(sp.multiply(sp.exp(x), g)),
+                                            sp.sum(sp.multiply(sp.exp(x), g))),
+        "mean": lambda x, g: sp.mean(sp.multiply(sp.sigmoid(x), g)),
+        "no product": lambda x, g: sp.sum(sp.square(x)),
+        "axis": lambda x, g: sp.sum(sp.sum(sp.multiply(sp.gelu(x), g), [0, 1], True)),
+    }
+    for name, loss in losses.items():
+        results = []
+        for hand_overs in (True, False):
+            sp.set_autograd_hand_overs(hand_overs)
+            try:
+                x, g = tensor(a, True), tensor(c)
+                for _ in range(2):  # the second pass accumulates
+                    loss(x, g).backward()
+                results.append(x.grad().to(sp.Device.cpu()).numpy())
+            finally:
+                sp.set_autograd_hand_overs(True)
+            assert_bitexact(g.to(sp.Device.cpu()).numpy(), c, f"{name}: the operand")
+        assert_bitexact(results[0], results[1], name)
