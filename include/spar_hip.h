@@ -538,6 +538,14 @@ struct SparHipStatus spar_hip_launch_cross_entropy_forward(
     uint64_t classes, uint64_t sequence_length, int dtype, int target_dtype, int language_model,
     int device);
 
+/* The same, with *invalid_target in host memory.  Waits for the check of the
+ * targets, not for the losses.  Refused on a stream under capture. */
+struct SparHipStatus spar_hip_cross_entropy_forward(
+    int32_t* invalid_target, void* losses, void* row_max, void* row_log_sum,
+    int32_t* undefined_rows, const void* logits, const void* targets, uint64_t logits_rows,
+    uint64_t classes, uint64_t sequence_length, int dtype, int target_dtype, int language_model,
+    int device);
+
 /* Its backward: logits_gradient = g - exp(lp) * g_t with g the NLL gradient
  * (g_t = 0 - loss_gradient at the target, zero elsewhere) and lp recomputed
  * from the saved row statistics -- the reference's nll_gradient followed by

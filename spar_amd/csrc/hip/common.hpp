@@ -71,6 +71,23 @@ SparHipStatus finish(const DeviceGuard& guard);
 hipError_t scratch_allocate(void** pointer, uint64_t bytes, int device);
 void scratch_release(void* pointer, int device);
 
+// A 32-bit word of pinned host memory that kernels write to, with the event
+// that says they have: the host waits for the kernel that sets the word, not
+// for what was launched after it.  Each caller holds a word of its own (any
+// thread); a device keeps up to kHostFlagsKept for the next callers.
+constexpr size_t kHostFlagsKept = 16;
+
+struct HostFlag {
+  int32_t* word = nullptr;        // host address
+  int32_t* device_word = nullptr; // its device address
+  hipEvent_t event = nullptr;
+};
+
+// The guard's device is current for both.  A flag is released only when no
+// launched kernel can write it any more.
+hipError_t host_flag_acquire(HostFlag& flag, int device);
+void host_flag_release(const HostFlag& flag, int device);
+
 // ------------------------------------------------------------- geometry
 
 // Fast unsigned division by an invariant divisor, following Granlund &

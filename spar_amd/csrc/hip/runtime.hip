@@ -34,6 +34,8 @@ struct DeviceState {
   std::multimap<uint64_t, void*> free_blocks;       // size -> block
   std::unordered_map<void*, uint64_t> live_blocks;  // block -> size
   SparHipMemoryStats stats{};
+  HostFlag free_flags[kHostFlagsKept];
+  size_t free_flag_count = 0;
 };
 
 std::mutex g_devices_mutex;
@@ -220,6 +222,60 @@ hipError_t scratch_allocate(void** pointer, uint64_t bytes, int device) {
 void scratch_release(void* pointer, int device) {
   DeviceState* state = state_for(device);
   if (state != nullptr && pointer != nullptr) release_on(state, pointer);
+}
+
+namespace {
+
+void host_flag_destroy(const HostFlag& flag) {
+  if (flag.event != nullptr) static_cast<void>(hipEventDestroy(flag.event));
+  if (flag.word != nullptr) static_cast<void>(hipHostFree(flag.word));
+}
+
+}  // namespace
+
+hipError_t host_flag_acquire(HostFlag& flag, int device) {
+  DeviceState* state = state_for(device);
+  if (state == nullptr) return hipErrorInvalidDevice;
+  {
+    std::lock_guard<std::mutex> lock(state->mutex);
+    if (state->free_flag_count > 0) {
+      flag = state->free_flags[--state->free_flag_count];
+      return hipSuccess;
+    }
+  }
+  HostFlag made;
+  void* word = nullptr;
+  void* device_word = nullptr;
+  hipError_t error =
+      hipHostMalloc(&word, sizeof(int32_t), hipHostMallocMapped | hipHostMallocCoherent);
+  if (error == hipSuccess) {
+    made.word = static_cast<int32_t*>(word);
+    error = hipHostGetDevicePointer(&device_word, word, 0);
+  }
+  if (error == hipSuccess) {
+    made.device_word = static_cast<int32_t*>(device_word);
+    error = hipEventCreateWithFlags(&made.event, hipEventDisableTiming);
+  }
+  if (error != hipSuccess) {
+    host_flag_destroy(made);
+    static_cast<void>(hipGetLastError());
+    return error;
+  }
+  flag = made;
+  return hipSuccess;
+}
+
+void host_flag_release(const HostFlag& flag, int device) {
+  DeviceState* state = state_for(device);
+  if (state == nullptr) return;
+  {
+    std::lock_guard<std::mutex> lock(state->mutex);
+    if (state->free_flag_count < kHostFlagsKept) {
+      state->free_flags[state->free_flag_count++] = flag;
+      return;
+    }
+  }
+  host_flag_destroy(flag);
 }
 
 }  // namespace spar_hip

@@ -74,24 +74,20 @@ Tensor fused_nll(const Tensor& logits, const Tensor& targets, Shape output_shape
   Tensor row_max{row_shape, logits.dtype(), device};
   Tensor row_log_sum{row_shape, logits.dtype(), device};
   Tensor undefined{row_shape, DType::Int32, device};
-  Tensor invalid{Shape{1}, DType::Int32, device};
   const int dtype{hip::dtype_tag(logits.dtype())};
   const int target_dtype{hip::dtype_tag(snapshot.dtype())};
   const int language_model{sequence_length == 0 ? 0 : 1};
-  hip::check(spar_hip_launch_cross_entropy_forward(
-                 HipTensorAccess::mutable_data(losses), HipTensorAccess::mutable_data(row_max),
-                 HipTensorAccess::mutable_data(row_log_sum),
+  // Target validation (cross_entropy.cpp:141, cuda_ops.cppm:550-566) waits for
+  // the check of the targets, as the reference's does; the losses are still
+  // being computed when it returns.
+  std::int32_t invalid_target{0};
+  hip::check(spar_hip_cross_entropy_forward(
+                 &invalid_target, HipTensorAccess::mutable_data(losses),
+                 HipTensorAccess::mutable_data(row_max), HipTensorAccess::mutable_data(row_log_sum),
                  static_cast<std::int32_t*>(HipTensorAccess::mutable_data(undefined)),
-                 static_cast<std::int32_t*>(HipTensorAccess::mutable_data(invalid)),
                  HipTensorAccess::data(x), HipTensorAccess::data(snapshot), rows, classes,
                  sequence_length, dtype, target_dtype, language_model, device.index()),
              "cross_entropy forward", device);
-  // Target validation (cross_entropy.cpp:141, cuda_ops.cppm:550-566) reads
-  // the device flag back, which synchronises, as the reference's does.
-  std::int32_t invalid_target{0};
-  hip::check(spar_hip_copy_device_to_host(&invalid_target, HipTensorAccess::data(invalid),
-                                          sizeof(invalid_target), device.index()),
-             "cross_entropy target validation", device);
   if (invalid_target != 0) {
     throw std::out_of_range{"cross_entropy target is outside the class range"};
   }

@@ -123,6 +123,8 @@ SIGNATURES = {
     "spar_hip_launch_nll_backward": [_P, _P, _P, _U64, _U64, _U64, _I, _I, _I, _I],
     "spar_hip_launch_cross_entropy_forward": [_P, _P, _P, _P, _P, _P, _P, _U64, _U64, _U64, _I, _I,
                                               _I, _I],
+    "spar_hip_cross_entropy_forward": [ctypes.POINTER(ctypes.c_int32), _P, _P, _P, _P, _P, _P,
+                                       _U64, _U64, _U64, _I, _I, _I, _I],
     "spar_hip_launch_cross_entropy_backward": [_P, _P, _P, _P, _P, _P, _P, _U64, _U64, _U64, _I,
                                                _I, _I, _I],
     "spar_hip_gradient_norm_summary": [ctypes.POINTER(NormSummary), _P, _U64, _I, _I],

@@ -216,6 +216,67 @@ def test_cross_entropy_errors(sp):
     assert float(sp.loss.cross_entropy(logits, ok).to(sp.Device.cpu()).numpy()) == pytest.approx(np.log(3))
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("batch,sequence", [(1, 2), (3, 257), (64, 4099)])
+def test_target_check_covers_every_target(sp, dtype, batch, sequence):
+    """The check runs ahead of the losses, over more targets than its grid
+    has lanes in the last shape: the first, a middle and the last target are
+    each found; the language-model form passes over each sequence's first
+    token, which is no target."""
+    device = sp.Device.hip(0)
+    classes = 3
+    logits = sp.Tensor.from_numpy(np.zeros((batch, sequence, classes), F32)).to(device)
+    ids = np.ones((batch, sequence), dtype)
+    used = [(0, 1), (batch // 2, sequence // 2), (batch - 1, sequence - 1)]
+
+    def losses(name, values):
+        tensor = sp.Tensor.from_numpy(values).to(device)
+        return getattr(sp.loss, name)(logits, tensor, sp.loss.Reduction.None_).to(
+            sp.Device.cpu()).numpy()
+
+    for name in ("cross_entropy", "language_model_cross_entropy"):
+        for where in used:
+            for bad in (-1, classes):
+                values = ids.copy()
+                values[where] = bad
+                with pytest.raises(IndexError, match="outside the class range"):
+                    losses(name, values)
+        assert np.allclose(losses(name, ids), np.log(3.0), rtol=1e-6)
+    values = ids.copy()
+    values[:, 0] = classes
+    assert np.allclose(losses("language_model_cross_entropy", values), np.log(3.0), rtol=1e-6)
+    with pytest.raises(IndexError):
+        losses("cross_entropy", values)
+
+
+def test_target_checks_of_several_threads(sp):
+    """Each caller waits for a flag of its own: eight threads, half of them
+    with a bad target."""
+    import threading
+
+    device = sp.Device.hip(0)
+    logits = sp.Tensor.from_numpy(np.zeros((4096, 5), F32)).to(device)
+    good = np.zeros(4096, np.int64)
+    bad = good.copy()
+    bad[4095] = 5
+    found = [0] * 8
+
+    def work(index):
+        targets = sp.Tensor.from_numpy(bad if index % 2 else good).to(device)
+        for _ in range(25):
+            try:
+                sp.loss.cross_entropy(logits, targets)
+            except IndexError:
+                found[index] += 1
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert found == [25 * (i % 2) for i in range(8)]
+
+
 # ------------------------------------------------ reference-compatible ABI
 
 def test_validate_targets(hip):
