@@ -401,6 +401,17 @@ struct SparHipStatus spar_hip_launch_multiply_reduce(
     const uint64_t* gradient_extents, uint64_t original_rank, const uint64_t* original_extents,
     uint64_t count, int dtype, int device);
 
+/* The same, and both gradients of a product gradient_shape x original_shape at
+ * once where one pass can write them: product[i] = gradient[i] * original
+ * [element i broadcasts from] (contiguous, the gradient's shape; `original`
+ * contiguous, original_extents).  *product_written says whether it was written;
+ * the destination always is, with the same sums as above. */
+struct SparHipStatus spar_hip_launch_multiply_backward(
+    void* destination, const void* gradient, const void* factor, uint64_t gradient_rank,
+    const uint64_t* gradient_extents, uint64_t original_rank, const uint64_t* original_extents,
+    uint64_t count, const void* original, void* product, int* product_written, int dtype,
+    int device);
+
 /* --------------------------------------------------------------- softmax */
 
 /* Softmax (logarithmic = 0) or log-softmax (1) over slices (outer, axis,

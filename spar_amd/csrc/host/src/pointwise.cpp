@@ -5,6 +5,7 @@
 #include <cmath>
 #include <limits>
 #include <optional>
+#include <utility>
 
 #include "autograd_internal.hpp"
 #include "bridge.hpp"
@@ -98,6 +99,35 @@ Tensor multiply_then_reduce(const Tensor& gradient, const Tensor& factor, const 
     return result;
   }
   return detail::reduce_gradient_to_shape(multiply(gradient, factor), shape);
+}
+
+// Both gradients of a product of `full`, which has the output's shape, and
+// `small`, which was broadcast: (gradient * small, reduction of gradient *
+// full).  Where one pass writes both, the gradient is read once; the values
+// are those of the separate passes.
+std::pair<Tensor, Tensor> product_gradients(const Tensor& gradient, const Tensor& full,
+                                            const Tensor& small) {
+  if (gradient.numel() != 0 && full_contiguous(gradient, full.shape()) &&
+      full.is_contiguous() && small.is_contiguous() &&
+      gradient.shape() == detail::broadcast_shape(gradient.shape(), small.shape())) {
+    Tensor reduced{small.shape(), gradient.dtype(), gradient.device()};
+    Tensor product{full.shape(), gradient.dtype(), gradient.device()};
+    const auto gradient_extents{hip::extents_of(gradient.shape())};
+    const auto small_extents{hip::extents_of(small.shape())};
+    int written{0};
+    hip::check(spar_hip_launch_multiply_backward(
+                   HipTensorAccess::mutable_data(reduced), HipTensorAccess::data(gradient),
+                   HipTensorAccess::data(full), gradient_extents.size(), gradient_extents.data(),
+                   small_extents.size(), small_extents.data(), gradient.numel(),
+                   HipTensorAccess::data(small), HipTensorAccess::mutable_data(product), &written,
+                   hip::dtype_tag(gradient.dtype()), gradient.device().index()),
+               "multiply backward", gradient.device());
+    if (written != 0) return {std::move(product), std::move(reduced)};
+    product = Tensor{Shape{}, gradient.dtype(), Device::cpu()};  // its block is free again
+    return {multiply(gradient, small), std::move(reduced)};
+  }
+  Tensor product{multiply_then_reduce(gradient, small, full.shape())};
+  return {std::move(product), multiply_then_reduce(gradient, full, small.shape())};
 }
 
 std::vector<Tensor> requiring(const Tensor& a, const Tensor& b, bool grad_a, bool grad_b) {
@@ -245,6 +275,15 @@ Tensor multiply(const Tensor& a, const Tensor& b) {
         output, requiring(a, b, grad_a, grad_b),
         [grad_a, grad_b, shape_a, shape_b, saved_a, saved_b](const Tensor& gradient) {
           std::vector<Tensor> contributions;
+          if (grad_a && grad_b && shape_a != shape_b &&
+              (shape_a == gradient.shape() || shape_b == gradient.shape())) {
+            const bool a_full{shape_a == gradient.shape()};
+            auto [product, reduced]{a_full ? product_gradients(gradient, *saved_a, *saved_b)
+                                           : product_gradients(gradient, *saved_b, *saved_a)};
+            contributions.push_back(std::move(a_full ? product : reduced));
+            contributions.push_back(std::move(a_full ? reduced : product));
+            return contributions;
+          }
           if (grad_a) contributions.push_back(multiply_then_reduce(gradient, *saved_b, shape_a));
           if (grad_b) contributions.push_back(multiply_then_reduce(gradient, *saved_a, shape_b));
           return contributions;

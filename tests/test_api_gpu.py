@@ -837,3 +837,32 @@ def test_autograd_ones_handed_through_products(sp, dtype):
                 sp.set_autograd_hand_overs(True)
             assert_bitexact(g.to(sp.Device.cpu()).numpy(), c, f"{name}: the operand")
         assert_bitexact(results[0], results[1], name)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,small", [((4, 64, 256), (4, 1, 256)), ((30, 2048), (2048,)),
+                                         ((6, 5, 7), (5, 7)), ((9, 12), (9, 1)),
+                                         ((3, 4), (1, 3, 4)), ((7, 8), ())])
+def test_autograd_product_of_a_broadcast_operand(sp, dtype, shape, small):
+    """Both gradients of a product with a broadcast operand, in either order
+    of the operands, are those of products with one tracked operand each."""
+    rng = np.random.default_rng(73)
+    device, cpu = sp.Device.hip(0), sp.Device.cpu()
+    x, s, g = (rng.standard_normal(n).astype(dtype) for n in (shape, small, shape))
+    swap_shape = np.broadcast_shapes(shape, small)
+
+    def gradients(tracked, swapped):
+        t = {}
+        for name, values in (("x", x), ("s", s)):
+            t[name] = sp.Tensor.from_numpy(values).to(device)
+            if name in tracked:
+                t[name].set_requires_grad(True)
+        y = sp.multiply(t["s"], t["x"]) if swapped else sp.multiply(t["x"], t["s"])
+        weight = sp.Tensor.from_numpy(g.reshape(swap_shape)).to(device)
+        sp.sum(sp.multiply(sp.add_scalar(y, 0.5), weight)).backward()
+        return [t[name].grad().to(cpu).numpy() for name in tracked]
+
+    for swapped in (False, True):
+        both = gradients(("x", "s"), swapped)
+        assert_bitexact(both[0], gradients(("x",), swapped)[0], "dx")
+        assert_bitexact(both[1], gradients(("s",), swapped)[0], "ds")

@@ -1071,6 +1071,51 @@ def test_broadcast_reduce_and_product(hip, dtype, gshape, oshape):
     assert_red(out.to_numpy(dtype, oshape), want, n, norm, f"multiply_reduce {gshape}->{oshape}")
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("gshape,oshape,written", [
+    ((4, 64, 256), (4, 1, 256), True),       # waves interleave the rows
+    ((3, 1, 8), (3, 1, 8), False),           # nothing is reduced
+    ((5, 4), (4,), True), ((1025, 12), (12,), True), ((2, 3, 37, 20), (2, 3, 1, 20), True),
+    ((300, 2048), (2048,), True),            # wide rows, a group a lane, split
+    ((2, 33, 4096), (2, 1, 4096), True),     # four groups a lane, remainders
+    ((67, 16384), (1, 16384), True),
+    ((700, 1028), (1028,), True),            # wide rows with an idle tail
+    ((6, 50, 7), (6, 1, 7), False),          # rows of no whole groups
+    ((64, 48), (64, 1), False), ((8, 16, 32), (1, 16, 1), False), ((8, 16, 32), (1,), False),
+])
+def test_multiply_backward_pair(hip, dtype, gshape, oshape, written):
+    """The second product written beside the sums: its bits are multiply's, the
+    sums' bits those of the sum alone, and a call that has no such pass (or
+    whose buffers are off 16 bytes) says so and leaves the product alone."""
+    import ctypes
+
+    rng = np.random.default_rng(91)
+    g, f = (rng.standard_normal(gshape).astype(dtype) for _ in range(2))
+    g.flat[0], g.flat[1] = np.inf, -0.0
+    o = rng.standard_normal(oshape).astype(dtype)
+    o.flat[0] = 0.0
+    gd, fd, od = (dev(hip, v) for v in (g, f, o))
+    alone = out_buf(hip, oshape, dtype)
+    shapes = (len(gshape), hip.u64_array(gshape), len(oshape), hip.u64_array(oshape), g.size)
+    hip.call("spar_hip_launch_multiply_reduce", alone.ptr, gd.ptr, fd.ptr, *shapes, tag(dtype), 0)
+    with np.errstate(invalid="ignore"):
+        want = g * o
+    for shift in (0, 1):  # an element past a 16-byte boundary
+        product = dev(hip, np.full(g.size + 1, 7, dtype))
+        sums = out_buf(hip, oshape, dtype)
+        flag = ctypes.c_int(7)
+        hip.call("spar_hip_launch_multiply_backward", sums.ptr, gd.ptr, fd.ptr, *shapes, od.ptr,
+                 product.ptr + shift * np.dtype(dtype).itemsize, ctypes.byref(flag), tag(dtype), 0)
+        assert flag.value == int(written and shift == 0)
+        assert_bitexact(sums.to_numpy(dtype, oshape), alone.to_numpy(dtype, oshape), "sums")
+        got = product.to_numpy(dtype, (g.size + 1,))
+        if flag.value:
+            assert_bitexact(got[:-1].reshape(gshape), want, "product")
+            assert got[-1] == 7
+        else:
+            assert np.all(got == 7)
+
+
 # --------------------------------------------------------------- softmax
 
 def softmax_device(hip, x, outer, extent, inner, log, dtype):
