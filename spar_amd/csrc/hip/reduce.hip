@@ -1613,7 +1613,10 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
       // the second product: `a` is read once for both, with the same splits
       // and so the same sums.  The affine
       // step [32, 1024, 4096] float32 (dscale 163 us and dx 159 us before) went
-      // from 1060 to 1019 us, [4, 64, 256] from 44.4 to 41.3 us.
+      // from 1060 to 1019 us, [4, 64, 256] from 44.4 to 41.3 us.  (With the
+      // next rows' loads ahead of these rows' stores, in two register sets, the
+      // large step took 1023 us; with one group a lane and four times the
+      // waves 1128.)
       if constexpr (K == Kind::Sum && NIN == 2) {
         if (beside.out != nullptr && vec && !multi && aligned16(beside.factor) &&
             aligned16(beside.out)) {
