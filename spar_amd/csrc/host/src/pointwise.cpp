@@ -104,11 +104,13 @@ Tensor multiply_then_reduce(const Tensor& gradient, const Tensor& factor, const 
 // Both gradients of a product of `full`, which has the output's shape, and
 // `small`, which was broadcast: (gradient * small, reduction of gradient *
 // full).  Where one pass writes both, the gradient is read once; the values
-// are those of the separate passes.
+// are those of the separate passes.  With exact zero signs on the separate
+// passes run: reduce_gradient_to_shape then adds +0 to the first, which the
+// one pass does not.
 std::pair<Tensor, Tensor> product_gradients(const Tensor& gradient, const Tensor& full,
                                             const Tensor& small) {
-  if (gradient.numel() != 0 && full_contiguous(gradient, full.shape()) &&
-      full.is_contiguous() && small.is_contiguous() &&
+  if (!exact_gradient_zero_signs() && gradient.numel() != 0 &&
+      full_contiguous(gradient, full.shape()) && full.is_contiguous() && small.is_contiguous() &&
       gradient.shape() == detail::broadcast_shape(gradient.shape(), small.shape())) {
     Tensor reduced{small.shape(), gradient.dtype(), gradient.device()};
     Tensor product{full.shape(), gradient.dtype(), gradient.device()};

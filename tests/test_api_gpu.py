@@ -322,6 +322,33 @@ def test_exact_gradient_zero_signs(sp):
         sp.set_exact_gradient_zero_signs(False)
 
 
+@pytest.mark.parametrize("small", [(4,), (2, 1), (1, 4), (3, 1, 4), (1,)])
+@pytest.mark.parametrize("order", ["full first", "small first"])
+def test_exact_zero_signs_of_broadcast_products(sp, small, order):
+    """The full operand's gradient of a broadcast product, gradient * small, is
+    added to +0 as well, whether or not one pass could write both gradients:
+    with a negative gradient its elements at small's zeros are +0.0."""
+    full = (3, 2, 4)
+    a = normal(44, full)
+    s = normal(45, small)
+    s.reshape(-1)[0] = 0.0
+    w = -np.abs(normal(46, full))
+
+    def build(lib, t):
+        product = lib.multiply(t[0], t[1]) if order == "full first" else lib.multiply(t[1], t[0])
+        # at small's zeros the product's gradient is -2 * w * w
+        return lib.sum(lib.multiply(lib.square(lib.add(product, t[2])), t[3]))
+
+    sp.set_exact_gradient_zero_signs(True)
+    try:
+        _, _, gd, gr = run_both(sp, build, [a, s, w, -w])
+        zeros = np.broadcast_to(s, full) == 0
+        assert zeros.any() and (gr[0][zeros] == 0).all() and not np.signbit(gr[0][zeros]).any()
+        assert_bitexact(gd[0], gr[0], "the full operand's gradient")
+    finally:
+        sp.set_exact_gradient_zero_signs(False)
+
+
 def test_autograd_unary_chain(sp):
     x = normal(15, (8, 32))
     w = normal(16, (8, 32))
