@@ -696,7 +696,10 @@ __global__ void __launch_bounds__(kLoopThreads)
 // Units are numbered over (outer, inner), so a small inner extent still fills
 // the lanes.  Slots past the axis are skipped (the test is the same for all
 // lanes).
+// Launches are split into grids of at most kMaxGrid workgroups (a launch of
+// 2^32 work-items is refused), each with its own first unit.
 struct SliceUnits {
+  uint64_t first;     // first unit of this launch
   uint64_t units;     // outer x units per block of slices
   uint64_t per_outer; // ceil(inner / G)
   uint64_t axis;
@@ -712,7 +715,7 @@ struct SliceUnit {
 
 template <int G, int X>
 __device__ __forceinline__ SliceUnit slice_unit(const SliceUnits& s) {
-  const uint64_t unit = static_cast<uint64_t>(blockIdx.x) * X + threadIdx.x % X;
+  const uint64_t unit = s.first + static_cast<uint64_t>(blockIdx.x) * X + threadIdx.x % X;
   if (unit >= s.units) return SliceUnit{0, 0, 0};
   const uint64_t o = unit / s.per_outer;
   const uint64_t i = (unit - o * s.per_outer) * G;
@@ -1175,7 +1178,12 @@ void launch_slices(uint64_t outer, uint64_t axis, uint64_t inner, const DeviceGu
         if (S::E != 0 && axis > static_cast<uint64_t>(S::Y) * S::E) return false;
         const uint64_t per_outer = (inner + S::G - 1) / S::G;
         const uint64_t units = outer * per_outer;
-        launch(shape, nt, SliceUnits{units, per_outer, axis, inner}, (units + S::X - 1) / S::X);
+        constexpr uint64_t kMost = kMaxGrid * S::X;
+        for (uint64_t first = 0; first < units; first += kMost) {
+          const uint64_t count = units - first < kMost ? units - first : kMost;
+          launch(shape, nt, SliceUnits{first, units, per_outer, axis, inner},
+                 static_cast<uint32_t>((count + S::X - 1) / S::X));
+        }
         return true;
       }
       return false;
@@ -1219,17 +1227,15 @@ void forward(void* output, int32_t* undefined, const void* input, uint64_t outer
     return;
   }
   launch_slices<T, 1>(outer, axis, inner, guard, [&](auto shape, auto nt, const SliceUnits& units,
-                                           uint64_t grid) {
+                                           uint32_t grid) {
     using S = decltype(shape);
     constexpr bool NT = decltype(nt)::value;
     if constexpr (S::E == 0) {
       forward_slice_loop_kernel<T, S::G, S::X, S::Y, LOG, NT>
-          <<<static_cast<uint32_t>(grid), S::X * S::Y, 0, guard.stream>>>(out, undefined, in,
-                                                                          units);
+          <<<grid, S::X * S::Y, 0, guard.stream>>>(out, undefined, in, units);
     } else {
       forward_slice_kernel<T, S::G, S::X, S::Y, S::E, LOG, NT>
-          <<<static_cast<uint32_t>(grid), S::X * S::Y, 0, guard.stream>>>(out, undefined, in,
-                                                                          units);
+          <<<grid, S::X * S::Y, 0, guard.stream>>>(out, undefined, in, units);
     }
   });
 }
@@ -1251,17 +1257,15 @@ void backward(void* output, const void* gradient, const void* saved, const int32
     return;
   }
   launch_slices<T, 2>(outer, axis, inner, guard, [&](auto shape, auto nt, const SliceUnits& units,
-                                           uint64_t grid) {
+                                           uint32_t grid) {
     using S = decltype(shape);
     constexpr bool NT = decltype(nt)::value;
     if constexpr (S::E == 0) {
       backward_slice_loop_kernel<T, S::G, S::X, S::Y, LOG, NT>
-          <<<static_cast<uint32_t>(grid), S::X * S::Y, 0, guard.stream>>>(out, g, y, undefined,
-                                                                          units);
+          <<<grid, S::X * S::Y, 0, guard.stream>>>(out, g, y, undefined, units);
     } else {
       backward_slice_kernel<T, S::G, S::X, S::Y, S::E, LOG, NT>
-          <<<static_cast<uint32_t>(grid), S::X * S::Y, 0, guard.stream>>>(out, g, y, undefined,
-                                                                          units);
+          <<<grid, S::X * S::Y, 0, guard.stream>>>(out, g, y, undefined, units);
     }
   });
 }

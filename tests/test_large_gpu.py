@@ -15,6 +15,10 @@ switches to 64-bit coordinates where a count or a row count passes
   * a sum over the unit axis of [2^31 + 16, 1] (2^31 + 16 rows: the
     reduction's 64-bit row map).
 
+Softmax along a short axis takes more workgroups than one launch may have:
+[2, 2^32] over its first axis (2^32 work-items, 103 GB with its gradients) and
+[2^22 + 1, 2, 17] over its middle one, forward and backward.
+
 Elementwise results are compared with the oracle on windows at the start,
 across element 2^31 and at the end; the full sum within red(N) of a float64
 sum of every element.  Before each launch the largest offset the launch can
@@ -24,7 +28,7 @@ import numpy as np
 import pytest
 
 from oracle import ops as ref
-from tests.helpers import assert_bitexact, assert_red
+from tests.helpers import assert_bitexact, assert_red, assert_ulp
 
 pytestmark = pytest.mark.gpu
 
@@ -121,3 +125,38 @@ def test_row_map_past_2_31_rows(hip, big):
         x = window(hip, a, start, count, shape=(count, 1))
         assert_bitexact(window(hip, out, start, count), ref.axis_sum(x, [1]),
                         f"unit-axis sum at row {start}")
+
+
+@pytest.mark.parametrize("outer,axis,inner", [(1, 2, 1 << 32), ((1 << 22) + 1, 2, 17)])
+def test_softmax_slices_past_one_launch(hip, outer, axis, inner):
+    count, slices = outer * axis * inner, outer * inner
+    x, g, y, dx = (hip.DeviceBuffer(count * 4) for _ in range(4))
+    flags = hip.DeviceBuffer(slices * 4)
+    try:
+        for buffer, seed in ((x, 74), (g, 75)):
+            hip.call("spar_hip_random_normal", buffer.ptr, count, hip.FLOAT32, seed, 0.0, 1.0, 0)
+        hip.call("spar_hip_launch_probability_forward", y.ptr, flags.ptr, x.ptr, outer, axis, inner,
+                 hip.FLOAT32, 0, 0)
+        hip.call("spar_hip_launch_probability_backward", dx.ptr, g.ptr, y.ptr, flags.ptr, outer,
+                 axis, inner, hip.FLOAT32, 0, 0)
+        # around the launches' first slices (2^20 workgroups of 64 slices), the
+        # middle and the end
+        width = 40
+        for start in (0, (1 << 26) - 20, slices // 2, 63 * (1 << 26) - 20, slices - width):
+            if start + width > slices:
+                continue
+            at = [((o * axis + a) * inner + i) for o, i in
+                  (divmod(start + k, inner) for k in range(width)) for a in range(axis)]
+            xs, gs, ys, dxs = (np.concatenate([window(hip, buffer, k, 1) for k in at])
+                               .reshape(width, axis) for buffer in (x, g, y, dx))
+            want, _ = ref.softmax_axis(xs, 1)
+            assert_ulp(ys, want, 4, f"softmax slices at {start}")
+            exact = ys * (gs - (gs * ys).sum(1, keepdims=True, dtype=np.float64))
+            # a product, the sum of two, a difference and a product, rounded
+            bound = 8 * 2.0 ** -24 * np.abs(gs).sum(1, keepdims=True)
+            assert (np.abs(dxs - exact) <= bound).all(), f"gradient of slices at {start}"
+            assert (window(hip, flags, start, width, np.int32) == 0).all()
+    finally:
+        for buffer in (x, g, y, dx, flags):
+            buffer.free()
+        hip.call("spar_hip_empty_cache", 0)
