@@ -1245,6 +1245,37 @@ __global__ void __launch_bounds__(kThreads)
 
 // ------------------------------------------------------------------ planner
 
+// What the three kernels over several reduced axes take, in microseconds past
+// what all share, fitted to 868 sums and argmaxes of 2^16 to 2^23 elements
+// ([A, K, R] and [A, K, B, C] over axes 0 and 2, float32 and float64; within a
+// third for most).  No one size tells them apart: a wave per output is bound
+// by its 64-lane steps of 64-bit divisions (0.55 us each, 0.22 ns where the
+// waves fill the chip), a workgroup per output by its barriers (1.8 ns, 3 with
+// indices) and the lines it gathers, the columns by rows of however few lanes
+// (0.069 ns a wave) and by the second launch of their splits.  With the waves
+// / here, float32 sums over axes 0 and 2: [2, 1000000, 4] 276 / 1797 us,
+// [3, 20000, 64] 16 / 42, [8, 2048, 256] 22 / 7, [24, 96, 3136] 759 / 12
+// (runs); [8, 4096, 256, 2] 53 / 626, [4, 128, 64, 32] 9 / 15,
+// [16, 2048, 16, 16] 31 / 51, [16, 1024, 16, 32] 43 / 36,
+// [4, 32, 64, 1000] 44 / 15 (columns).
+struct SeveralAxesCost {
+  static double waves(uint64_t outputs, uint64_t count) {
+    const double steps = static_cast<double>((count + kWave - 1) / kWave);
+    return steps * 0.22e-3 * static_cast<double>(outputs > 2500 ? outputs : 2500);
+  }
+  static double runs(uint64_t outputs, uint64_t splits, uint64_t bytes, uint64_t run_bytes,
+                     bool indexed) {
+    const double lines = static_cast<double>(bytes / run_bytes) * ((run_bytes + 127) / 128);
+    const double workgroups = static_cast<double>(outputs) * static_cast<double>(splits);
+    return workgroups * (indexed ? 3.0e-3 : 1.8e-3) +
+           static_cast<double>(outputs) * lines * 16e-6 + (splits > 1 ? 5.0 : 0.0);
+  }
+  static double columns(uint64_t column_blocks, uint64_t rows, uint64_t splits) {
+    return 6.0 + 0.069e-3 * static_cast<double>(column_blocks) *
+                     static_cast<double>(rows + 24 * splits);
+  }
+};
+
 // A reduction over a permuted, coalesced view: kept axes (output order) and
 // reduced axes (flattened-index order), each innermost last.
 struct Plan {
@@ -1397,6 +1428,24 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     }
   }
 
+  // One wave per output, any layout.
+  auto one_wave_per_output = [&]() -> hipError_t {
+    const RowMap map = make_row_map(plan, plan.kept_rank);
+    ReducedMap red{};
+    red.rank = plan.red_rank;
+    red.count = plan.reduced;
+    for (int k = 0; k < plan.red_rank; ++k) {
+      red.extents[k] = plan.red_extents[plan.red_rank - 1 - k];
+      red.strides[k] = plan.red_strides[plan.red_rank - 1 - k];
+    }
+    generic_kernel<T, K, NIN><<<grid_for((plan.outputs + kWaves - 1) / kWaves), kThreads, 0,
+                                guard.stream>>>(a, b, plan.outputs, map, red, final_sink());
+    return hipSuccess;
+  };
+  // What that takes over several reduced axes, to weigh against the runs' and
+  // the columns' kernels: see SeveralAxesCost.
+  const double wave_cost = SeveralAxesCost::waves(plan.outputs, plan.reduced);
+
   if (plan.red_rank == 0) {
     // Nothing is reduced (all reduced extents are 1): a reduction of one
     // element per output.
@@ -1506,6 +1555,11 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     }
     const uint64_t segment = ((count + splits - 1) / splits + width - 1) / width * width;
     splits = (count + segment - 1) / segment;
+    const uint64_t run_bytes = plan.red_extents[plan.red_rank - 1] * sizeof(T);
+    if (wave_cost < SeveralAxesCost::runs(outputs, splits, count * sizeof(T), run_bytes,
+                                          K == Kind::Max)) {
+      return one_wave_per_output();
+    }
     auto launch = [&](const Sink<T>& s) {
       auto kernel = vec ? run_kernel<T, K, NIN, true> : run_kernel<T, K, NIN, false>;
       kernel<<<grid_for(outputs * splits), kThreads, 0, guard.stream>>>(a, b, outputs, count,
@@ -1596,6 +1650,10 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     }
     // several reduced axes never asked for a workspace: one split needs none
     if (multi && shape.splits > most_splits) shape.splits = most_splits < 1 ? 1 : most_splits;
+    if (multi && wave_cost < SeveralAxesCost::columns(outer * shape.column_blocks, n,
+                                                      shape.splits)) {
+      return one_wave_per_output();
+    }
     const uint64_t column_blocks = shape.column_blocks;
     uint64_t splits = shape.splits;
     const uint64_t range_splits =
@@ -1724,18 +1782,7 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     }, value_only);
   }
 
-  // Generic: one wave per output.
-  const RowMap map = make_row_map(plan, plan.kept_rank);
-  ReducedMap red{};
-  red.rank = plan.red_rank;
-  red.count = plan.reduced;
-  for (int k = 0; k < plan.red_rank; ++k) {
-    red.extents[k] = plan.red_extents[plan.red_rank - 1 - k];
-    red.strides[k] = plan.red_strides[plan.red_rank - 1 - k];
-  }
-  generic_kernel<T, K, NIN><<<grid_for((plan.outputs + kWaves - 1) / kWaves), kThreads, 0,
-                              guard.stream>>>(a, b, plan.outputs, map, red, final_sink());
-  return hipSuccess;
+  return one_wave_per_output();
 }
 
 template <typename T, int NIN>

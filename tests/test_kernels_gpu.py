@@ -742,6 +742,27 @@ def test_several_reduced_axes(hip, dtype, shape, order, axes):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [
+    (2, 5000, 16),         # runs: a wave per output, one 64-lane step
+    (3, 2048, 1), (2, 2048, 33), (64, 1000, 8), (64, 1000, 16), (8, 600, 256),  # either side
+    (8, 300, 256, 2),      # columns: a wave per output of few lanes
+    (16, 64, 16, 16), (16, 64, 16, 33), (4, 128, 64, 32), (8, 16, 512, 4), (4, 8, 64, 1000),
+])
+def test_several_reduced_axes_by_cost(hip, dtype, shape):
+    """Sums and maxima over axes 0 and 2 on both sides of the line between a
+    wave per output and the kernels for runs and columns."""
+    base = inputs(65, int(np.prod(shape)), dtype, with_specials=False).reshape(shape)
+    check_axis(hip, base, base, [0, 2], dtype, f"several axes {shape}")
+    spiked = np.round(base * 2)
+    spiked[-1, 1, 0] = np.nan
+    spiked[:, 2] = -np.inf
+    mx, am = ref.axis_max(spiked, [0, 2])
+    for op, want in (("max", mx), ("argmax", am)):
+        assert_bitexact(axis_reduce(hip, spiked, spiked, [0, 2], op, dtype), want,
+                        f"{op} with ties, NaNs and -inf {shape}")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(24, 96, 784), (3, 127, 3136), (2, 128, 3136), (5, 31, 4096)])
 def test_few_wide_rows(hip, dtype, shape):
     """Fewer than 128 wide rows on too few waves take the interleaved scan."""
