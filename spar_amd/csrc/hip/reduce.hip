@@ -1640,12 +1640,14 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     // Rows that are wide but too few to split well, in waves that do not fill
     // the chip, are interleaved as well, over four times the waves: the sum of
     // [24, 96, 3136] float32 over axis 1 took 17.1 us with 168 workgroups of
-    // 96-row waves and takes 8.0 us, of [32, 32, 8192] 13.8 and 8.1 us; from
-    // 128 rows or two workgroups of waves per CU on the wide scan is ahead.
-    // (A request that the fixed workspace refused stays refused.)
+    // 96-row waves and takes 8.0 us, of [32, 32, 8192] 13.8 and 8.1 us.  The
+    // wide scan is ahead from 128 rows on, past one of its workgroups per CU
+    // ([200, 100, 1024] float64, 400 of them: 28.1 us against 29.2), and under
+    // 32 rows ([200, 7, 1024] float32 maxima 7.8 us against 10.5) unless it
+    // would split 16 ([1, 24, 4096]: 8.3 us against 5.2).  (A request that the fixed workspace refused stays refused.)
     const uint64_t wide_blocks = outer * ((inner / W + kThreads - 1) / kThreads);
-    if (shape.wide && n < 128 && wide_blocks < static_cast<uint64_t>(cus) * 2 &&
-        shape.splits <= most_splits) {
+    if (shape.wide && n < 128 && n >= (shape.quad ? 16 : 32) &&
+        wide_blocks <= static_cast<uint64_t>(cus) && shape.splits <= most_splits) {
       shape = shape_of(false);
     }
     // several reduced axes never asked for a workspace: one split needs none

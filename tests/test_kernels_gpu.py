@@ -763,7 +763,9 @@ def test_several_reduced_axes_by_cost(hip, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("shape", [(24, 96, 784), (3, 127, 3136), (2, 128, 3136), (5, 31, 4096)])
+@pytest.mark.parametrize("shape", [(24, 96, 784), (3, 127, 3136), (2, 128, 3136), (5, 31, 4096),
+                                   (3, 31, 3136), (3, 32, 3136), (2, 15, 4096), (2, 16, 4096),
+                                   (256, 33, 1024), (257, 33, 1024)])
 def test_few_wide_rows(hip, dtype, shape):
     """Fewer than 128 wide rows on too few waves take the interleaved scan."""
     base = inputs(62, int(np.prod(shape)), dtype, with_specials=False).reshape(shape)
