@@ -348,9 +348,16 @@ __device__ __forceinline__ SliceStats<T> row_stats(SliceStats<T> s) {
 // Waves per SIMD the register budget must allow: a row of up to 128 bytes
 // per lane (and a float32 odd row's one more element) fits in 64 VGPRs (8
 // waves, two 1024-lane workgroups per CU); longer rows get 128 (4 waves).
-template <typename T, int SLOTS>
+// Workgroups of up to 256 lanes whose rows are float64 of 128 bytes a lane, or
+// have that one more element, spill to scratch in 64 and get 80 (6 waves):
+// softmax of [32768, 600] float64 87.5 us in 64 and 58.2 in 80, log-softmax of
+// [8190, 4097] float32 51.3 and 45.7.
+template <typename T, int SLOTS, int L>
 constexpr int row_waves() {
-  return sizeof(T) * SLOTS <= 132 ? 8 : 4;
+  constexpr size_t bytes = sizeof(T) * SLOTS;
+  if (bytes < 128) return 8;
+  if (bytes <= 136 && L <= 256 && (sizeof(T) == 8 || SLOTS > 32)) return 6;
+  return bytes <= 132 ? 8 : 4;
 }
 
 template <int L>
@@ -360,7 +367,7 @@ constexpr int row_threads() {
 
 template <typename T, int L, int E, bool LOG, int LAYOUT, bool NT>
 __global__ void __launch_bounds__(row_threads<L>())
-    __attribute__((amdgpu_waves_per_eu(row_waves<T, kRowSlots<E, LAYOUT>>())))
+    __attribute__((amdgpu_waves_per_eu(row_waves<T, kRowSlots<E, LAYOUT>, L>())))
     forward_row_kernel(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n) {
   constexpr int W = Vec16<T>::width;
   constexpr int N = kRowSlots<E, LAYOUT>;
@@ -1109,11 +1116,16 @@ bool with_row_shape(uint64_t rows, uint64_t n, bool aligned, Launch&& launch, Sh
 // Row lengths up to 1024 take one wave or part of one per row (no cross-wave
 // exchange; rows of 8 to 128 were one to a wave and took 14.4 us for 49152 of
 // them, 4.6-8.3 us several to a wave); 8192 takes 256 lanes x 32, which
-// measured faster than 512 x 16.  Up to 65536 float32 stay in registers: 512
-// rows of 50257 take 76 us, where three scalar reads of each took 140 us.
+// measured faster than 512 x 16.  Float64 rows of 8193 to 16384 take 512 lanes
+// x 32 (in 1024 x 16 the odd ones need more than 64 VGPRs: log-softmax of
+// [4095, 8193] 147 us there, 106 so), float32 rows up to 24576 have a shape of
+// their own (odd ones spill in 1024 x 32: log-softmax of [1677, 20001] 52.1 us
+// there, 45.6 so).  Up to 65536 float32 stay in registers: 512 rows of 50257
+// take 76 us, where three scalar reads of each took 140 us.
 template <typename T, bool LOG>
 bool launch_forward_rows(T* out, int32_t* undefined, const T* in, uint64_t rows, uint64_t n,
                          const DeviceGuard& guard) {
+  constexpr bool kSingle = sizeof(T) == 4;
   return with_row_shape<T>(
       rows, n, aligned16(out) && aligned16(in),
       [&](auto shape, auto layout, auto nt, uint64_t first, uint64_t count, uint32_t grid) {
@@ -1123,8 +1135,10 @@ bool launch_forward_rows(T* out, int32_t* undefined, const T* in, uint64_t rows,
                                                              in + first * n, count, n);
       },
       RowShape<4, 4>{}, RowShape<8, 4>{}, RowShape<16, 4>{}, RowShape<32, 4>{}, RowShape<64, 4>{},
-      RowShape<64, 16>{}, RowShape<256, 16>{}, RowShape<256, 32>{}, RowShape<1024, 16>{},
-      RowShape<1024, 32>{}, RowShape<1024, sizeof(T) == 4 ? 64 : 32>{});
+      RowShape<64, 16>{}, RowShape<256, 16>{}, RowShape<256, 32>{},
+      RowShape<(kSingle ? 1024 : 512), (kSingle ? 16 : 32)>{},
+      RowShape<1024, (kSingle ? 24 : 32)>{}, RowShape<1024, 32>{},
+      RowShape<1024, (kSingle ? 64 : 32)>{});
 }
 
 template <typename T, bool LOG>

@@ -1314,7 +1314,8 @@ def test_softmax_rows_beyond_one_grid(hip):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 63, 65, 127, 129, 255, 257, 1023,
-                               1025, 4097, 8191, 16385, 32769, 65535, 65537])
+                               1025, 4097, 8191, 8193, 16383, 16385, 24575, 24576, 24577, 32769, 65535,
+                               65537])
 def test_softmax_odd_rows(hip, dtype, n):
     """Rows of any length from a misaligned start, several to a wave where
     they are short, with undefined rows beside defined ones: the register
