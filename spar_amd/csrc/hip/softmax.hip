@@ -469,6 +469,14 @@ __global__ void __launch_bounds__(row_threads<L>())
     }
   }
   const T reduced = row_sum<T, L>(local);
+  // (A select per element, in place of the branch, had every exponential
+  // computed ahead of the first store.)
+  if (bad) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) g[j] = quiet_nan<T>();
+    store_row<T, L, E, LAYOUT, NT>(out + r * n, g, n, live);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     if constexpr (LOG) {
@@ -476,7 +484,6 @@ __global__ void __launch_bounds__(row_threads<L>())
     } else {
       g[j] = y[j] * (g[j] - reduced);
     }
-    if (bad) g[j] = quiet_nan<T>();
   }
   store_row<T, L, E, LAYOUT, NT>(out + r * n, g, n, live);
 }
