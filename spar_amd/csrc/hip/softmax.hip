@@ -1182,6 +1182,18 @@ struct SliceShape {
 // registers (a 1024-lane workgroup has 128), and longer axes are looped.
 constexpr uint64_t kWideInner = 32;
 
+// Short axes take as few row groups as hold them: lanes without a row, and the
+// logarithm or reciprocal that every row group computes for itself, cost more
+// than a longer column of registers.  Log-softmax forward of [1000, 2, 1000]
+// float64 took 15.5 us with a lane per slice, 27.8 with four row groups and
+// takes 12.9 with one; of [1000, 5, 1000] 25.5, 34.4 with four and 22.4 with
+// two; of [1000, 17, 1000] 85.4, 116 with 16 and 50 with four.  From about 20
+// rows on (24 float64), or where the slices do not fill the chip, 16 row groups
+// are ahead of four (softmax of [1000, 28, 1000] float32 1.1 times, of
+// [16, 24, 512] 1.2 times as fast).
+template <typename T>
+constexpr uint64_t kQuarterRows = sizeof(T) == 4 ? 20 : 24;
+
 // Long axes of few slices (workgroups for less than a quarter of the CUs) take
 // a quarter of the slices per workgroup and more row groups: softmax of
 // [4, 1000, 256] float32 over axis 1 took 17.0 us in 16 workgroups and takes
@@ -1222,7 +1234,11 @@ void launch_slices(uint64_t outer, uint64_t axis, uint64_t inner, const DeviceGu
       return;
     }
     if (vectors) {
-      as(SliceShape<W, 16, 4, 4>{}) || as(SliceShape<W, 16, 16, 4>{}) ||
+      const bool full = groups >= static_cast<uint64_t>(guard.multiprocessors) * 4;
+      as(SliceShape<W, 64, 1, 4>{}) || as(SliceShape<W, 32, 2, 4>{}) ||
+          as(SliceShape<W, 16, 4, 4>{}) ||
+          (full && axis <= kQuarterRows<T> && as(SliceShape<W, 16, 4, 8>{})) ||
+          as(SliceShape<W, 16, 16, 4>{}) ||
           as(SliceShape<W, 16, 32, 8>{}) || as(SliceShape<W, 16, 64, 8>{}) ||
           as(SliceShape<W, 16, 64, 16>{}) || as(SliceShape<W, 16, 64, 0>{});
     } else {

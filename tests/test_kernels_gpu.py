@@ -1375,7 +1375,10 @@ SLICE_SHAPES = [(3, 1, 40), (2, 16, 32), (3, 17, 33), (2, 64, 47), (2, 65, 64), 
                 (2, 257, 66), (1, 512, 100), (300, 513, 36), (1, 1025, 35), (1, 2048, 33),
                 (1, 2049, 34), (200, 300, 64), (130, 1100, 40), (5, 16, 2), (7, 17, 31),
                 (3, 64, 5), (2, 65, 7), (2, 257, 3), (1, 1024, 30), (1, 1025, 2), (1, 2100, 9),
-                (2000, 300, 3), (3000, 520, 2), (2500, 1030, 3)]
+                (2000, 300, 3), (3000, 520, 2), (2500, 1030, 3),
+                # short axes: one, two and four row groups
+                (3, 2, 257), (2, 4, 300), (3, 5, 131), (2, 8, 129), (2, 9, 66), (1100, 17, 64),
+                (1100, 20, 63), (1100, 21, 64), (2200, 24, 64), (2200, 25, 64)]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
