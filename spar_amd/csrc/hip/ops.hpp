@@ -87,27 +87,19 @@ __device__ __forceinline__ double math_sqrt(double x) { return sqrt(x); }
 __device__ __forceinline__ float math_tanh(float x) { return tanhf(x); }
 __device__ __forceinline__ double math_tanh(double x) { return tanh(x); }
 
-// exp rounded once from double precision: (float)exp((double)x) is the
-// correctly rounded float32 exponential except when exp(x) lies within about
-// 2^-47 (relative) of a float32 rounding boundary.  glibc's expf, which the
-// CPU path calls, is correctly rounded in the same sense, so composite ops
-// built on it (sigmoid, silu) reproduce the CPU's float operations.  The
-// arguments here are never positive: a Cody-Waite reduction by ln 2 and the
-// degree-11 Taylor polynomial on |r| <= ln(2)/2 (truncation 6.3e-15) replace
-// the library's double exp, whose range tests and table-free full-precision
-// polynomial, run once for each branch of the sigmoid, kept silu at 2.3 TB/s:
-// [2047, 2731] float32 took 19.4 us and takes 12.8 us, [8192, 4096] 85.8 and
-// 53.0 us.  Below -110 the float32 result is 0; NaN propagates (the compare is
-// false).
-__device__ __forceinline__ float rounded_exp_nonpositive(float x) {
+// exp(y) for -110 <= y <= 0 in double, within an ulp (2^-52): a Cody-Waite
+// reduction by ln 2 and the degree-13 Taylor polynomial on |r| <= ln(2)/2
+// (truncation 2^-57).
+__host__ __device__ __forceinline__ double accurate_exp_nonpositive(double y) {
   constexpr double kLog2e = 0x1.71547652b82fep0;
   constexpr double kLn2High = 0x1.62e42fefa39efp-1;
   constexpr double kLn2Low = 0x1.abc9e3b39803fp-56;
-  const double y = x < -110.0f ? -110.0 : static_cast<double>(x);
   const double k = __builtin_rint(y * kLog2e);
   double r = __builtin_fma(-k, kLn2High, y);
   r = __builtin_fma(-k, kLn2Low, r);
-  double p = 1.0 / 39916800.0;
+  double p = 1.0 / 6227020800.0;
+  p = __builtin_fma(p, r, 1.0 / 479001600.0);
+  p = __builtin_fma(p, r, 1.0 / 39916800.0);
   p = __builtin_fma(p, r, 1.0 / 3628800.0);
   p = __builtin_fma(p, r, 1.0 / 362880.0);
   p = __builtin_fma(p, r, 1.0 / 40320.0);
@@ -119,7 +111,23 @@ __device__ __forceinline__ float rounded_exp_nonpositive(float x) {
   p = __builtin_fma(p, r, 0.5);
   p = __builtin_fma(p, r, 1.0);
   p = __builtin_fma(p, r, 1.0);
-  return static_cast<float>(__builtin_ldexp(p, static_cast<int>(k)));
+  return __builtin_ldexp(p, static_cast<int>(k));
+}
+
+// exp rounded once from double precision: (float)exp((double)x) is the
+// correctly rounded float32 exponential except when exp(x) lies within about
+// 2^-52 (relative) of a float32 rounding boundary.  glibc's expf, which the
+// CPU path calls, is correctly rounded in the same sense, so composite ops
+// built on it (sigmoid, silu) reproduce the CPU's float operations.  The
+// arguments here are never positive, which spares the library's double exp its
+// range tests: with it, run once for each branch of the sigmoid, silu of [2047,
+// 2731] float32 took 18.2 us and of [8192, 4096] 78.0; they take 12.1 and 51.1
+// (11.8 and 49.0 with a degree-11 polynomial, whose 2^-47 rounds a few
+// exponentials the other way).  Below -110 the float32 result is 0; NaN
+// propagates (the compare is false).
+__host__ __device__ __forceinline__ float rounded_exp_nonpositive(float x) {
+  return static_cast<float>(
+      accurate_exp_nonpositive(x < -110.0f ? -110.0 : static_cast<double>(x)));
 }
 __device__ __forceinline__ double rounded_exp_nonpositive(double x) { return exp(x); }
 
