@@ -5,16 +5,17 @@
 // ceil(rows/256) blocks (32 for 8192 rows) and read each row three times.
 // Semantics follow the CPU path (src/ops/softmax.cpp:42-150, :342-444).
 //
-// CDNA4 design for the last axis (inner == 1), the common case: one
-// workgroup per row holds the whole row in VGPRs (up to 32768 float32 with
-// 1024 lanes x 8 float4), so the row is read from HBM once and written once:
-//   pass over registers 1: first-occurrence max;
-//   workgroup combine through wave64 shuffles and a 16-entry LDS exchange;
+// CDNA4 design for the last axis (inner == 1), the common case: part of a
+// wave, a wave or a workgroup holds the whole row in VGPRs (up to 65536 float32
+// or 32768 float64 forward, 32768 of either backward), so the row is read from
+// HBM once and written once:
+//   pass over registers 1: the maximum;
+//   combine through wave64 shuffles and, past a wave, an LDS exchange;
 //   pass 2: e = exp(x - max), sum; pass 3: p = e / sum (log: (x-max) - log sum).
-// A row's workgroup stays under 64 VGPRs per lane, so two or more rows share
-// a CU and one row's loads overlap another's reductions and stores.
-// Backward keeps g and y (or log p) in registers the same way.  Rows longer
-// than the register budget take a three-read loop.  A non-last axis
+// Rows of up to 128 bytes per lane take 64 to 80 VGPRs, so two or more
+// workgroups share a CU and one row's loads overlap another's reductions and
+// stores; longer rows take 128.  Backward keeps g and y (or log p) in registers
+// the same way.  Longer rows are read twice in each direction.  A non-last axis
 // (inner > 1) keeps its slices in registers too, spread over the lanes of a
 // workgroup by rows and by neighbouring slices.
 #include <hip/hip_runtime.h>
@@ -29,8 +30,10 @@ namespace {
 
 constexpr uint64_t kMaxGrid = uint64_t{1} << 20;
 
-// Statistics of a slice: first-occurrence maximum (value and 32-bit column;
-// rows are far shorter than 2^31), NaN flag, +inf count.
+// Statistics of a slice: first-occurrence maximum (value and 32-bit column),
+// NaN flag, +inf count.  The column only orders equal maxima, which is of no
+// consequence to the values taken from here, so it may wrap on a slice of 2^31
+// elements or more.
 template <typename T>
 struct SliceStats {
   T value;
@@ -539,8 +542,10 @@ __device__ __forceinline__ void block_online(T& m, T& s) {
 // Rows past the register budget, 16 bytes per lane at element alignment, four
 // in flight; the n % W last elements go to the first lanes.  The forward keeps
 // a running maximum and rescaled exp-sum per lane and reads the row again for
-// the results: softmax of [256, 70001] float32 takes 38 us, where three scalar
-// reads took 98 us.
+// the results: softmax of [256, 70001] float32 takes 40 us, where three scalar
+// reads took 88 us (three wide ones take 46).  The rescaling costs no
+// precision: the sum's mean relative error over 12288 rows of 70001 is 5.13e-8
+// (+-0.03e-8) both ways.
 constexpr int kLoopThreads = 1024;
 constexpr int kLoopBatch = 4;
 
@@ -1333,14 +1338,6 @@ struct TargetMap {
 
 constexpr int kEntropyThreads = 256;
 
-// Row statistics in one streaming pass, branch-free: each lane keeps a
-// running maximum m and s = sum exp(x - m); per batch of 8 vectors it takes
-// the batch maximum (v_max, which passes over NaN), rescales s once by
-// exp(m - m_new) and adds exp(x - m_new) per element, where a -inf element
-// adds exactly 0 (as it does to a row with a finite maximum).  A NaN element
-// makes s NaN (NaN - m) and a +inf maximum does too (inf - inf); a row of
-// nothing above -inf keeps m = -inf.  Only the sign of a zero maximum can
-// differ from the first-occurrence rule, which changes no loss or gradient.
 // A row's target, where its loss goes and the logit there.
 template <typename T>
 struct RowTarget {
@@ -1393,8 +1390,7 @@ struct LossOutputs {
   }
 };
 
-// 16 bytes of a logits row: non-temporal from aligned rows, cached from rows
-// of odd length (ODD).
+// 16 bytes of a logits row, at element alignment for rows of odd length (ODD).
 template <typename T, bool ODD>
 __device__ __forceinline__ typename Vec16<T>::type class_group(const T* at) {
   if constexpr (ODD) {
@@ -1404,9 +1400,16 @@ __device__ __forceinline__ typename Vec16<T>::type class_group(const T* at) {
   }
 }
 
-// Forward: one streaming pass per logits row (non-temporal 16-byte loads at
-// element alignment, batches of eight per lane) gives the row maximum m and S = sum exp(x - m);
-// then loss = -((x_t - m) - log S), the log-softmax value at the target
+// Forward: one streaming pass per logits row (non-temporal 16-byte loads,
+// batches of eight per lane) gives the row maximum m and S = sum exp(x - m).
+// Branch-free: each lane keeps a running maximum m and s = sum exp(x - m); per
+// batch it takes the batch maximum (v_max, which passes over NaN), rescales s
+// once by exp(m - m_new) and adds exp(x - m_new) per element, where a -inf
+// element adds exactly 0 (as it does to a row with a finite maximum).  A NaN
+// element makes s NaN (NaN - m) and a +inf maximum does too (inf - inf); a row
+// of nothing above -inf keeps m = -inf.  Only the sign of a zero maximum can
+// differ from the first-occurrence rule, which changes no loss or gradient.
+// Then loss = -((x_t - m) - log S), the log-softmax value at the target
 // negated, with log-softmax's operations.  S carries the rescaling roundings
 // of the online sum (a few ulp; log-softmax's tolerance covers it).  The
 // target and its logit are fetched at the start of the row.  Saves m and
