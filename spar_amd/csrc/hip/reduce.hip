@@ -538,9 +538,10 @@ __device__ __forceinline__ Acc<T, K> group_reduce(Acc<T, K> acc) {
 }
 
 // Rows of kNarrowRow to kShortRow elements: L lanes per row (L a power of two
-// up to the wave, chosen so that a lane has one to four vectors), kThreads / L
-// rows per workgroup, combined by shuffles alone.  A workgroup per row left
-// most of its lanes without a load and spent two barriers on each row.  Loads
+// up to the wave: one or two vectors a lane in rows of up to 128 vectors, up to
+// four, float64 eight, in longer ones), kThreads / L rows per workgroup,
+// combined by shuffles alone.  A workgroup per row left most of its lanes
+// without a load and spent two barriers on each row.  Loads
 // are 16 bytes at element alignment, so odd lengths take them too; the n % W
 // last elements go to the group's first lanes.  Sums of 2^24 float32 elements
 // in rows of 49 / 64 / 256 / 1000 took 331 / 286 / 75 / 23.1 us with a
@@ -1466,8 +1467,7 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
       return hipSuccess;
     }
     if (n <= kShortRow) {
-      // lanes per row: about two vectors each, all of a wave from 256 elements
-      // (float32) on
+      // lanes per row: at most two vectors each, all of a wave past 64 vectors
       auto launch = [&](auto lanes) {
         constexpr int L = decltype(lanes)::value;
         constexpr uint64_t kRows = kThreads / L;
@@ -1644,14 +1644,16 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
     // wide scan is ahead from 128 rows on, past one of its workgroups per CU
     // ([200, 100, 1024] float64, 400 of them: 28.1 us against 29.2), and under
     // 32 rows ([200, 7, 1024] float32 maxima 7.8 us against 10.5) unless it
-    // would split 16 ([1, 24, 4096]: 8.3 us against 5.2).  (A request that the fixed workspace refused stays refused.)
+    // would split 16 ([1, 24, 4096]: 8.3 us against 5.2).  (A request that the
+    // fixed workspace refused stays refused.)
     const uint64_t wide_blocks = outer * ((inner / W + kThreads - 1) / kThreads);
     if (shape.wide && n < 128 && n >= (shape.quad ? 16 : 32) &&
         wide_blocks <= static_cast<uint64_t>(cus) && shape.splits <= most_splits) {
       shape = shape_of(false);
     }
-    // several reduced axes never asked for a workspace: one split needs none
-    if (multi && shape.splits > most_splits) shape.splits = most_splits < 1 ? 1 : most_splits;
+    // (The splits of several reduced axes always fit the fixed workspace: they
+    // make fewer than 16 workgroups per CU, of at most 2 KiB of partials each,
+    // less than 8 MiB on 256 CUs.)
     if (multi && wave_cost < SeveralAxesCost::columns(outer * shape.column_blocks, n,
                                                       shape.splits)) {
       return one_wave_per_output();
@@ -1671,9 +1673,9 @@ hipError_t run_plan(const Plan& plan, const T* a, const T* b, void* output, int 
       const uint32_t grid = grid_for(outer * splits * column_blocks);
       // Over one reduced axis and 16-byte groups the sum of products writes
       // the second product: `a` is read once for both, with the same splits
-      // and so the same sums.  The affine
-      // step [32, 1024, 4096] float32 (dscale 163 us and dx 159 us before) went
-      // from 1060 to 1019 us, [4, 64, 256] from 44.4 to 41.3 us.  (With the
+      // and so the same sums.  The affine step [32, 1024, 4096] float32 (dscale
+      // 163 us and dx 159 us before) went from 1060 to 1019 us, [4, 64, 256]
+      // from 44.4 to 41.3 us.  (With the
       // next rows' loads ahead of these rows' stores, in two register sets, the
       // large step took 1023 us; with one group a lane and four times the
       // waves 1128.)

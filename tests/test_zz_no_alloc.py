@@ -109,25 +109,30 @@ def test_no_alloc_layouts(hip, op):
 
 
 def test_no_alloc_keeps_several_axes_within_the_workspace(hip):
-    # Column sums over two axes that do not merge never needed a workspace:
-    # [256, 2, 4, 1024, 128] over axes 0 and 2 has 262,144 float64 outputs,
-    # whose splits would take 4 MiB (argmax 3 MiB) each, so they are capped to
-    # what fits.
-    shape = [256, 2, 4, 1024, 128]
-    x = normal(hip, int(np.prod(shape)), 36, np.float32)
-    strides = [2 * 4 * 1024 * 128, 4 * 1024 * 128, 1024 * 128, 128, 1]
-    say(f"no_alloc MAX, ARGMAX, SUM {shape} axes 0, 2")
-    host = x.to_numpy(np.float32, shape)
-    for op in ("MAX", "ARGMAX"):
+    # Reductions over axes that do not merge never needed a workspace, and their
+    # splits always fit it: columns are split where they make fewer than 8
+    # workgroups per CU, into less than 16 per CU.  The most partials are those
+    # of 8 * cus - 1 workgroups of 256 float32 columns, split in two: for
+    # max and argmax 2 KiB of values and indices each, 8,384,512 bytes of the
+    # 8 MiB on 256 CUs.
+    blocks = 8 * hip.multiprocessor_count() - 1
+    partials = 2 * blocks * 256 * (4 + 4)
+    assert partials + 256 <= 8 << 20
+    shape = [16, blocks, 8, 256]  # axes 0 and 2: 128 rows, two splits of 64
+    count = int(np.prod(shape))
+    x = normal(hip, count, 36, np.float32)
+    strides = [blocks * 8 * 256, 8 * 256, 256, 1]
+    for op in OPS:
+        say(f"no_alloc {op} {shape} axes 0, 2")
         want, got = run_both(hip, x, shape, strides, 0, 5, np.float32, getattr(hip, op))
         assert_bitexact(got, want, f"{op} {shape}")
-        if op == "MAX":
-            assert_bitexact(got, host.max(axis=(0, 2)).reshape(-1), "MAX of numpy")
-    # sums: the splits, and so the order, may differ between the entry points
+    host = x.to_numpy(np.float32, shape)
+    want, got = run_both(hip, x, shape, strides, 0, 5, np.float32, hip.MAX)
+    assert_bitexact(got, host.max(axis=(0, 2)).reshape(-1), "MAX of numpy")
     want, got = run_both(hip, x, shape, strides, 0, 5, np.float32, hip.SUM)
     exact = host.sum(axis=(0, 2), dtype=np.float64).reshape(-1)
-    bound = 1024 * 2.0 ** -24 * np.abs(host).sum(axis=(0, 2), dtype=np.float64).reshape(-1)
-    assert (np.abs(got - exact) <= bound).all() and (np.abs(want - exact) <= bound).all()
+    bound = 128 * 2.0 ** -24 * np.abs(host).sum(axis=(0, 2), dtype=np.float64).reshape(-1)
+    assert (np.abs(got - exact) <= bound).all()
 
 
 def test_no_alloc_refuses_plans_beyond_the_workspace(hip):
