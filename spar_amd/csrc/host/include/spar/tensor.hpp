@@ -304,9 +304,11 @@ void record_transfer_operation(Tensor& output, Tensor requiring_parent, Backward
 /// accumulations done in place or out of place, narrows whose gradient was
 /// handed to the narrow below them unembedded (a chain of narrows is
 /// embedded once), gradients a rule wrote straight into the gradient of
-/// a narrow chain's base (no embedding pass at all), and product gradients
-/// handed to a scaled rule as factor and value (no product pass).  The
-/// engine never copies an intermediate gradient.
+/// a narrow chain's base (no embedding pass at all), product gradients
+/// handed to a scaled rule as factor and value (no product pass), and
+/// products under the seed's ones whose input was handed the other operand
+/// (no product pass either).  The engine never copies an intermediate
+/// gradient.
 struct AutogradCounters final {
   std::uint64_t backward_calls;
   std::uint64_t leaf_copies;
@@ -315,6 +317,7 @@ struct AutogradCounters final {
   std::uint64_t window_fusions;
   std::uint64_t placed_gradients;
   std::uint64_t scaled_gradients;
+  std::uint64_t factor_gradients;
 };
 [[nodiscard]] AutogradCounters autograd_counters() noexcept;
 /// Process-wide: whether backward() hands gradients down narrow chains,

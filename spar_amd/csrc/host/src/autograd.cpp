@@ -32,8 +32,8 @@
 //      rounding and operand order, so x's producer computes what it would
 //      from the materialised product, and every identity still receives its
 //      gradients in the same order.
-//   7. A sweep starts from ones, and a sum hands its input the gradient it
-//      gets, broadcast.  Where the gradient of a product with one tracked
+//   7. A sweep starts from ones, and a sum to one element hands its input the
+//      gradient it gets, broadcast.  Where the gradient of a product with one tracked
 //      input is therefore known to be all ones, that input's gradient is the
 //      other operand itself (1 * v is v, bit for bit): it is handed on, and no
 //      product is formed.  The ones themselves are written only when a rule
@@ -69,6 +69,7 @@ std::atomic<std::uint64_t> g_out_of_place_adds{0};
 std::atomic<std::uint64_t> g_window_fusions{0};
 std::atomic<std::uint64_t> g_placed_gradients{0};
 std::atomic<std::uint64_t> g_scaled_gradients{0};
+std::atomic<std::uint64_t> g_factor_gradients{0};
 // Whether backward() may take the hand-overs of contract points 5 and 6
 // (narrow chains, placed gradients, scaled products); without them every
 // rule runs in its plain form, which the contract says gives the same bits.
@@ -157,7 +158,8 @@ void record_transfer_operation(Tensor& output, Tensor requiring_parent, Backward
 AutogradCounters autograd_counters() noexcept {
   return AutogradCounters{g_backward_calls.load(), g_leaf_copies.load(), g_in_place_adds.load(),
                           g_out_of_place_adds.load(), g_window_fusions.load(),
-                          g_placed_gradients.load(), g_scaled_gradients.load()};
+                          g_placed_gradients.load(), g_scaled_gradients.load(),
+                          g_factor_gradients.load()};
 }
 
 void set_autograd_hand_overs(bool enabled) noexcept {
@@ -465,6 +467,7 @@ class Sweep final {
       return false;
     }
     accumulate(input, factor.detach());
+    g_factor_gradients.fetch_add(1, std::memory_order_relaxed);
     return true;
   }
 

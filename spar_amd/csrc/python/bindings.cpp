@@ -342,6 +342,7 @@ PYBIND11_MODULE(_spar, m) {
     d["window_fusions"] = c.window_fusions;
     d["placed_gradients"] = c.placed_gradients;
     d["scaled_gradients"] = c.scaled_gradients;
+    d["factor_gradients"] = c.factor_gradients;
     return d;
   });
 }

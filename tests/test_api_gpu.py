@@ -826,7 +826,8 @@ def test_autograd_ones_handed_through_products(sp, dtype):
     """A product under plain sums hands its one tracked input the other
     operand, and the seed's ones are written only where a rule reads them: the
     gradients' bits are those of the plain rules, the operand itself is left
-    alone, and accumulated or shared gradients are not the operand's storage."""
+    alone, and accumulated or shared gradients are not the operand's storage.
+    The engine's counter says which losses took the hand-over."""
     rng = np.random.default_rng(71)
     device = sp.Device.hip(0)
     a, c = (rng.standard_normal((33, 65)).astype(dtype) for _ in range(2))
@@ -851,10 +852,13 @@ def test_autograd_ones_handed_through_products(sp, dtype):
         "no product": lambda x, g: sp.sum(sp.square(x)),
         "axis": lambda x, g: sp.sum(sp.sum(sp.multiply(sp.gelu(x), g), [0, 1], True)),
     }
+    # (the outer of two sums hands the inner a view of the ones, which is read)
+    handed = {"activation", "operand first", "passed on", "shared", "axis"}
     for name, loss in losses.items():
         results = []
         for hand_overs in (True, False):
             sp.set_autograd_hand_overs(hand_overs)
+            before = sp.autograd_counters()["factor_gradients"]
             try:
                 x, g = tensor(a, True), tensor(c)
                 for _ in range(2):  # the second pass accumulates
@@ -862,8 +866,63 @@ def test_autograd_ones_handed_through_products(sp, dtype):
                 results.append(x.grad().to(sp.Device.cpu()).numpy())
             finally:
                 sp.set_autograd_hand_overs(True)
+            taken = sp.autograd_counters()["factor_gradients"] - before
+            assert taken == (2 if hand_overs and name in handed else 0), name
             assert_bitexact(g.to(sp.Device.cpu()).numpy(), c, f"{name}: the operand")
         assert_bitexact(results[0], results[1], name)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_handed_operand_off_16_bytes(sp, dtype):
+    """The operand handed on as a gradient may be a contiguous view at any
+    element: every rule that may receive it gives the bits it gives with the
+    hand-overs off, whose gradients are dense tensors of their own.  (The norms
+    take the operand and the ones' value in a form of their own.)"""
+    rng = np.random.default_rng(72)
+    device = sp.Device.hip(0)
+    a = (np.abs(rng.standard_normal((32, 68))) + 0.1).astype(dtype)
+    base = rng.standard_normal(33 * 69).astype(dtype)
+    scale = rng.standard_normal((68,)).astype(dtype)
+    bias = rng.standard_normal((32, 1)).astype(dtype)
+    rules = {name: (lambda x, s, b, f=getattr(sp, name): f(x))
+             for name in ("silu", "sigmoid", "tanh", "gelu", "sqrt", "square", "reciprocal", "exp",
+                          "log", "negate")}
+    rules.update({
+        "softmax": lambda x, s, b: sp.softmax(x, 1),
+        "log-softmax slices": lambda x, s, b: sp.log_softmax(x, 0),
+        "broadcast product": lambda x, s, b: sp.multiply(x, s),
+        "broadcast sum": lambda x, s, b: sp.add(x, b),
+        "quotient": lambda x, s, b: sp.divide(s, x),
+        "scaled": lambda x, s, b: sp.multiply_scalar(x, 0.3),
+        "transposed": lambda x, s, b: sp.exp(sp.exp(x).transpose(0, 1).contiguous())
+                                        .transpose(0, 1).contiguous(),
+        "narrowed": lambda x, s, b: sp.exp(sp.add(x, b)).narrow(0, 0, 32),
+        "reshaped": lambda x, s, b: sp.exp(x).reshape([64, 34]).reshape([32, 68]),
+    })
+    for name, rule in rules.items():
+        results = []
+        for hand_overs in (True, False):
+            sp.set_autograd_hand_overs(hand_overs)
+            before = sp.autograd_counters()["factor_gradients"]
+            try:
+                leaves = [sp.Tensor.from_numpy(v).to(device) for v in (a, scale, bias)]
+                for leaf in leaves:
+                    leaf.set_requires_grad(True)
+                # 32 x 68 elements from element 69 on: contiguous, off 16 bytes
+                flat = sp.Tensor.from_numpy(base).to(device)
+                g = flat.narrow(0, 69, 32 * 68).reshape([32, 68])
+                assert g.is_contiguous()
+                sp.sum(sp.multiply(rule(*leaves), g)).backward()
+                results.append([leaf.grad().to(sp.Device.cpu()).numpy() if leaf.has_grad else None
+                                for leaf in leaves])
+            finally:
+                sp.set_autograd_hand_overs(True)
+            taken = sp.autograd_counters()["factor_gradients"] - before
+            assert taken == (1 if hand_overs else 0), name
+        for got, want in zip(*results):
+            assert (got is None) == (want is None), name
+            if got is not None:
+                assert_bitexact(got, want, name)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
