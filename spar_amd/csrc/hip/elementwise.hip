@@ -71,36 +71,18 @@ __global__ void __launch_bounds__(kVectorThreads)
     map2_vec_kernel(T* out, const T* a, const T* b, uint64_t count, F f) {
   using V = typename Vec16<T>::type;
   constexpr int W = Vec16<T>::width;
-  constexpr int U = VectorsPerLane<F>::value;
   const uint64_t vectors = count / W;
-  const uint64_t tile = static_cast<uint64_t>(kVectorThreads) * U;
   const V* a_v = reinterpret_cast<const V*>(a);
   const V* b_v = reinterpret_cast<const V*>(b);
   V* out_v = reinterpret_cast<V*>(out);
-  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * tile; base < vectors;
-       base += static_cast<uint64_t>(gridDim.x) * tile) {
-    V ra[U];
-    V rb[U];
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kVectorThreads + threadIdx.x; i < vectors;
+       i += static_cast<uint64_t>(gridDim.x) * kVectorThreads) {
+    const V va = stream_load(a_v + i);
+    const V vb = stream_load(b_v + i);
+    V o;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t i = base + static_cast<uint64_t>(u) * kVectorThreads + threadIdx.x;
-      if (i < vectors) {
-        ra[u] = stream_load(a_v + i);
-        rb[u] = stream_load(b_v + i);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint64_t i = base + static_cast<uint64_t>(u) * kVectorThreads + threadIdx.x;
-      if (i < vectors) {
-        V o;
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-          vec_set<T>(o, k, f(vec_get<T>(ra[u], k), vec_get<T>(rb[u], k)));
-        }
-        store_vector<NT>(out_v + i, o);
-      }
-    }
+    for (int k = 0; k < W; ++k) vec_set<T>(o, k, f(vec_get<T>(va, k), vec_get<T>(vb, k)));
+    store_vector<NT>(out_v + i, o);
   }
   if (blockIdx.x == 0) {
     const uint64_t i = vectors * W + threadIdx.x;
@@ -262,8 +244,8 @@ void launch_map2(T* out, const T* a, const T* b, uint64_t count, F f, const Devi
   if (aligned16(out) && aligned16(a) && aligned16(b)) {
     with_policy(stream_output(count * sizeof(T)), [&](auto nt) {
       map2_vec_kernel<T, F, decltype(nt)::value>
-          <<<vector_grid(count, Vec16<T>::width, VectorsPerLane<F>::value), kVectorThreads, 0,
-             guard.stream>>>(out, a, b, count, f);
+          <<<vector_grid(count, Vec16<T>::width), kVectorThreads, 0, guard.stream>>>(out, a, b,
+                                                                                    count, f);
     });
   } else {
     map2_scalar_kernel<T, F><<<scalar_grid(count, guard), kThreads, 0, guard.stream>>>(

@@ -357,7 +357,7 @@ __device__ __forceinline__ float gelu_derivative_float(float value) {
   return out;
 }
 
-// Ops with tens of fp64 operations per element take two vectors per lane
+// Unary ops with tens of fp64 operations per element take two vectors per lane
 // in the contiguous kernels, for more independent work per wave.
 template <typename F> struct VectorsPerLane { static constexpr int value = 1; };
 
