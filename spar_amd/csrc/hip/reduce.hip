@@ -1255,7 +1255,7 @@ __global__ void __launch_bounds__(kThreads)
 // indices) and the lines it gathers, the columns by rows of however few lanes
 // (0.069 ns a wave) and by the second launch of their splits.  With the waves
 // / here, float32 sums over axes 0 and 2: [2, 1000000, 4] 276 / 1797 us,
-// [3, 20000, 64] 16 / 42, [8, 2048, 256] 22 / 7, [24, 96, 3136] 759 / 12
+// [3, 20000, 64] 16 / 42, [8, 512, 256] 22 / 7, [24, 96, 3136] 759 / 12
 // (runs); [8, 4096, 256, 2] 53 / 626, [4, 128, 64, 32] 9 / 15,
 // [16, 2048, 16, 16] 31 / 51, [16, 1024, 16, 32] 43 / 36,
 // [4, 32, 64, 1000] 44 / 15 (columns).
